@@ -665,8 +665,9 @@ __global__ __launch_bounds__(NQ * NQ) void adv_diff_react_kernel(int nelmt, cons
                                                lds[0], lds[1], out + (size_t)e * NM * NM * NM, adv);
 }
 
-// Fused Helmholtz y = lambda*M x + L x (Helmholtz.h:549-599)
-template <typename T, int NM, int NQ, bool DEF, int EPB>
+// Fused Helmholtz y = lambda*M x + L x (Helmholtz.h:549-599), per-point
+// geometry (affine elements: hex_modal.hpp)
+template <typename T, int NM, int NQ, int EPB>
 __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_kernel(int nelmt, const T *__restrict__ tabp,
                                                                   const T *__restrict__ geo, T lambda,
                                                                   const T *__restrict__ in, T *__restrict__ out)
@@ -677,13 +678,13 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_kernel(int nelmt, con
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
     const int e = blockIdx.x * EPB + le;
     const bool valid = e < nelmt;
-    helmholtz_element<T, NM, NQ, DEF>(tab, LocalFetch<T, NM>{in + (size_t)e * NM * NM * NM}, valid, e, t, geo,
+    helmholtz_element<T, NM, NQ, true>(tab, LocalFetch<T, NM>{in + (size_t)e * NM * NM * NM}, valid, e, t, geo,
                                       lambda, lds[le][0], lds[le][1], out + (size_t)e * NM * NM * NM);
 }
 
 // Solver form on a general mesh: x gathered through the signed map from
 // the global vector, element results written element-major
-template <typename T, int NM, int NQ, bool DEF, int EPB>
+template <typename T, int NM, int NQ, int EPB>
 __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_mapped_kernel(int nelmt, const T *__restrict__ tabp,
                                                                          const T *__restrict__ geo, T lambda,
                                                                          const T *__restrict__ xg,
@@ -697,13 +698,13 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_mapped_kernel(int nel
     const int e = blockIdx.x * EPB + le;
     const bool valid = e < nelmt;
     const MappedFetch<T, NM> f{xg, menc + (size_t)(valid ? e : 0) * NM * NM * NM};
-    helmholtz_element<T, NM, NQ, DEF>(tab, f, valid, e, t, geo, lambda, lds[le][0], lds[le][1],
+    helmholtz_element<T, NM, NQ, true>(tab, f, valid, e, t, geo, lambda, lds[le][0], lds[le][1],
                                       out + (size_t)e * NM * NM * NM);
 }
 
 // Grouped form: several operators of the same kind in one launch; block b
 // belongs to the item whose [block0, next block0) range holds it.
-template <typename T, int NM, int NQ, bool DEF, int EPB>
+template <typename T, int NM, int NQ, int EPB>
 __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_grouped_kernel(int count,
                                                                           const GroupItem<T> *__restrict__ items,
                                                                           const T *__restrict__ tabp)
@@ -718,13 +719,13 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_grouped_kernel(int co
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
     const int e = (b - I.block0) * EPB + le;
     const bool valid = e < I.nelmt;
-    helmholtz_element<T, NM, NQ, DEF>(tab, LocalFetch<T, NM>{I.in + (size_t)e * NM * NM * NM}, valid, e, t, I.geo,
+    helmholtz_element<T, NM, NQ, true>(tab, LocalFetch<T, NM>{I.in + (size_t)e * NM * NM * NM}, valid, e, t, I.geo,
                                       I.lambda, lds[le][0], lds[le][1], I.out + (size_t)e * NM * NM * NM);
 }
 
 // Solver form: x gathered from the global vector of the structured n^3
 // mesh, element results written element-major (assembled afterwards).
-template <typename T, int NM, int NQ, bool DEF, int EPB>
+template <typename T, int NM, int NQ, int EPB>
 __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_gather_kernel(int n, int N, const T *__restrict__ tabp,
                                                                          const T *__restrict__ geo, T lambda,
                                                                          const T *__restrict__ xg,
@@ -741,7 +742,7 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_gather_kernel(int n, 
     const bool valid = e < nelmt;
     const int ex = e % n, ey = (e / n) % n, ez = e / (n * n);
     const StructuredFetch<T, NM> f{xg, N, ex * (NM - 1), ey * (NM - 1), ez * (NM - 1)};
-    helmholtz_element<T, NM, NQ, DEF>(tab, f, valid, e, t, geo, lambda, lds[le][0], lds[le][1],
+    helmholtz_element<T, NM, NQ, true>(tab, f, valid, e, t, geo, lambda, lds[le][0], lds[le][1],
                                       out + (size_t)e * NM * NM * NM);
 }
 

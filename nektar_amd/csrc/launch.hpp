@@ -91,8 +91,20 @@ constexpr int hex_fill_elems(int nq) { return 256 / (nq * nq) > 0 ? 256 / (nq * 
 // elements per 256-work-item workgroup; they are compiled for NUMMODES >=
 // kMfmaMinModes (where the per-direction products are dense enough).
 constexpr int kMfmaTile = 1024, kMfmaMinModes = 5;
-inline int hex_tile_elems(int nq, int tile)
+// Default of the Legendre-space kernels of affine elements (hex_modal.hpp,
+// NM^2 work-items per element): whole waves of one element (NM = 7, 8, 10)
+// or of as many as one wave or a few waves hold.  Measured in FP64 on 11.2 M
+// coefficients, best of 1, 2, 3, 4, 5, 7, 10 and 14 elements: NM = 3: 56 us
+// (1 element: 205), 4: 40 (118), 5: 49 (85), 6: 47 (59), 7: 49, 8: 42, 9: 51
+// (58), 10: 49; the same ones are best or within 3 % in FP32.
+constexpr int hex_modal_elems(int nm)
 {
+    return nm <= 4 ? 64 / (nm * nm) : nm <= 6 ? 5 : nm == 9 ? 2 : 1;
+}
+// elements per workgroup of a tile (0: the default) of a hex Helmholtz kind
+inline int hex_tile_elems(int nm, int nq, bool deformed, int tile)
+{
+    if (tile <= 0 && !deformed) return hex_modal_elems(nm);
     return tile >= kMfmaTile ? tile - kMfmaTile : (tile > 0 ? tile : hex_fill_elems(nq));
 }
 constexpr int tet_packed_tpe(int nq0) { return nq0 * (nq0 - 1); }
