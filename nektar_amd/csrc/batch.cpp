@@ -152,7 +152,8 @@ void Batch::build()
         for (int m : g.members) {
             const Entry &e = entries_[m];
             const MFOperator &o = *e.op;
-            const int nb = (o.nelmt + epb - 1) / epb;
+            const int nb = g.shape == Shape::Tet && !g.deformed ? tet_modal_blocks(o.nelmt)
+                                                                : (o.nelmt + epb - 1) / epb;
             if (g.fp32)
                 i32.push_back(GroupItem<float>{static_cast<const float *>(o.geo.get()),
                                                static_cast<const float *>(e.in), static_cast<float *>(e.out0),

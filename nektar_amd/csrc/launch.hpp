@@ -116,6 +116,18 @@ constexpr int tet_tile_elems(int nq0, int tile)
 {
     return 256 / (tile > 0 ? tile : tet_default_tpe(nq0)) > 0 ? 256 / (tile > 0 ? tile : tet_default_tpe(nq0)) : 1;
 }
+// Affine tets run the matrix-core kernel (tet_modal.hpp) whatever the tile:
+// 16 elements per wave, four waves per workgroup.  With `split` the four waves
+// share 16 elements: shorter, but more of it (each wave loads the 16 elements,
+// and the results are added through LDS).  Measured whole against split, FP64
+// us at 4,096 / 8,192 / 16,384 elements: NM = 4 4.0/3.4, 4.2/4.2, 4.8/5.9;
+// NM = 7 13/7.1, 14/11, 16/20; NM = 10 40/18, 42/32, 47/61; FP32 alike.  The
+// line lies where whole waves would fill five eighths of the 1024 SIMDs.
+constexpr bool tet_modal_split(int nelmt) { return nelmt <= 640 * 16; }
+constexpr int tet_modal_blocks(int nelmt)
+{
+    return tet_modal_split(nelmt) ? (nelmt + 15) / 16 : (nelmt + 63) / 64;
+}
 // tet tile candidates (work-items per element) in the order the autotuner
 // tries them
 int tet_tile_candidates(int nq0, int *out, int max);

@@ -5,6 +5,8 @@
 // (Collections/CoalescedGeomData.cpp:90-342).
 #include "mf_operator.hpp"
 
+#include "tet_modal_layout.hpp"
+
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -135,7 +137,9 @@ void MFOperator::init(const std::string &key, const int nummodes[3], const int n
                                                         : false);
     if (compiled) {
         ncoeff = num_coeffs(shape, nm);
-        tab.upload(build_tables(shape, nm, nq[0]), fp32);
+        tab.upload(shape == Shape::Tet && op == OpType::Helmholtz && !deformed ? tetmodal::build_tables(nm, fp32)
+                                                                               : build_tables(shape, nm, nq[0]),
+                   fp32);
     } else {
         NMF_REQUIRE(op != OpType::PhysInterp, NMF_ERR_UNSUPPORTED,
                     "PhysInterp1DScaled takes equal modes and the default points of the shape only");

@@ -882,7 +882,8 @@ __device__ __forceinline__ void helmholtz_block(int blk, int nelmt, const T *__r
     grad_transpose_to_coeffs<T, NM, NQ, TPE>(tab, lt, valid, t, e, y, v2, X, Y, out);
 }
 
-template <typename T, int NM, int NQ, bool DEF, int TPE>
+// per-point geometry (affine elements: tet_modal.hpp)
+template <typename T, int NM, int NQ, int TPE>
 __global__ __launch_bounds__((Tile<NM, NQ, TPE>::BLOCK), (kTetWaves<T, NQ>)) void helmholtz_kernel(int nelmt, const T *__restrict__ tabp,
                                                                             const T *__restrict__ geo, T lambda,
                                                                             const T *__restrict__ in,
@@ -892,7 +893,7 @@ __global__ __launch_bounds__((Tile<NM, NQ, TPE>::BLOCK), (kTetWaves<T, NQ>)) voi
     __shared__ T lds[Ti::EPB][2][Slab<T, NM, NQ>::SIZE];
     __shared__ __align__(16) T ltab[LTab<T, NM, NQ, kB2Global<T, NQ>>::SIZE];
     stage_tables<T, NM, NQ, kB2Global<T, NQ>>(tabp, ltab);
-    helmholtz_block<T, NM, NQ, DEF, TPE>(blockIdx.x, nelmt, tabp, geo, lambda, in, out, lds, ltab);
+    helmholtz_block<T, NM, NQ, true, TPE>(blockIdx.x, nelmt, tabp, geo, lambda, in, out, lds, ltab);
 }
 
 // LinearAdvectionDiffusionReaction (LinearAdvectionDiffusionReaction.h
@@ -916,7 +917,7 @@ __global__ __launch_bounds__((Tile<NM, NQ, TPE>::BLOCK)) void adv_diff_react_ker
 
 // Grouped form: several operators of the same kind in one launch; block b
 // belongs to the item whose [block0, next block0) range holds it.
-template <typename T, int NM, int NQ, bool DEF, int TPE>
+template <typename T, int NM, int NQ, int TPE>
 __global__ __launch_bounds__((Tile<NM, NQ, TPE>::BLOCK), (kTetWaves<T, NQ>)) void helmholtz_grouped_kernel(
     int count, const GroupItem<T> *__restrict__ items, const T *__restrict__ tabp)
 {
@@ -928,7 +929,7 @@ __global__ __launch_bounds__((Tile<NM, NQ, TPE>::BLOCK), (kTetWaves<T, NQ>)) voi
     int it = 0;
     while (it + 1 < count && b >= items[it + 1].block0) ++it;
     const GroupItem<T> I = items[it];
-    helmholtz_block<T, NM, NQ, DEF, TPE>(b - I.block0, I.nelmt, tabp, I.geo, I.lambda, I.in, I.out, lds, ltab);
+    helmholtz_block<T, NM, NQ, true, TPE>(b - I.block0, I.nelmt, tabp, I.geo, I.lambda, I.in, I.out, lds, ltab);
 }
 
 // IProductWRTDerivBase for tets (IProductWRTDerivBase.h:751-788, pointwise
