@@ -501,7 +501,7 @@ SolveInfo IterativeSolver::solve(double tol, int maxit)
             apply_from_global(w, yloc_.as<double>());
             map_.assemble(yloc_.as<double>(), s, stream_, true, w, pmu_.as<double>());
         }
-        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, pa_.as<double>(), pmu_.as<double>(), nb_));
+        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, pa_.as<double>(), nb_, pmu_.as<double>(), nb_));
         const int max_rounds = maxit / kItersPerChunk + 3;
         for (int round = 0;; ++round) {
             NMF_HIP(hipMemcpyAsync(host_state_, st, sizeof(solver::CGState), hipMemcpyDeviceToHost, stream_));
@@ -521,7 +521,7 @@ SolveInfo IterativeSolver::solve(double tol, int maxit)
                     apply_from_global(w, yloc_.as<double>());
                     map_.assemble(yloc_.as<double>(), s, stream_, true, w, pmu_.as<double>());
                 }
-                NMF_HIP(solver::launch_cg_scalar(stream_, st, pa_.as<double>(), pmu_.as<double>(), nb_));
+                NMF_HIP(solver::launch_cg_scalar(stream_, st, pa_.as<double>(), nb_, pmu_.as<double>(), nb_));
             }
         }
         NMF_HIP(hipEventRecord(e1, stream_));

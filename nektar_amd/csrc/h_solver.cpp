@@ -79,7 +79,7 @@ size_t HexSolver::estimate_bytes(int n, int nm, int nq, bool deformed, bool mixe
     const size_t N = (size_t)n * (nm - 1) + 1, NG = N * N * N, nel = (size_t)n * n * n;
     const size_t nloc = nel * nm * nm * nm;
     const size_t geo = nel * 7 * (deformed ? (size_t)nq * nq * nq : 1);
-    size_t b = 8 * (NG * (5 + 6) + nloc + geo);
+    size_t b = 8 * (NG * (5 + 5) + nloc + geo + nel);
     if (mixed) b += 4 * (NG * 7 + nloc + geo);
     b += 8 * nel * (size_t)nq * nq * nq;  // forcing / quadrature scratch
     // the small buffers, so that the estimate bounds device_bytes(): mesh
@@ -126,6 +126,7 @@ HexSolver::HexSolver(const HexBoxMesh &mesh, int nummodes, int numpoints, double
     for (auto *buf : {&b_, &x_, &invd_, &tmp64_, &r64_}) buf->allocate(NG_ * sizeof(double));
     sloc64_.allocate(nloc * sizeof(double));
     for (auto &v : cg64_) v.allocate(NG_ * sizeof(double));
+    edot_.allocate((size_t)nelmt_ * sizeof(double));
     state_.allocate(sizeof(CGState));
     // partial-sum buffers sized for the largest reduction grid any kernel uses
     pa_.allocate(3 * (size_t)solver::kRedBlocks * sizeof(double));
@@ -171,7 +172,7 @@ size_t HexSolver::device_bytes() const
 {
     size_t s = 0;
     for (const DeviceBuffer *b : {&X_, &z_, &w_, &tab64_, &tab32_, &dtab_, &geo64_, &geo32_, &b_, &x_, &invd_,
-                                  &invd32_, &sloc64_, &tmp64_, &r64_, &sloc32_, &state_, &pa_, &pmu_, &scalar_})
+                                  &invd32_, &sloc64_, &tmp64_, &r64_, &sloc32_, &state_, &pa_, &pmu_, &scalar_, &edot_})
         s += b->bytes();
     for (const auto &v : cg64_) s += v.bytes();
     for (const auto &v : cg32_) s += v.bytes();
@@ -231,7 +232,8 @@ void HexSolver::assemble_rhs(const double *f_dev)
 void HexSolver::apply_local(bool fp32, const void *xg, void *sloc, const int *done)
 {
     SolverArgs a{SolverKernel::Apply, fp32, deformed_, n_, N_, fp32 ? tab32_.get() : tab64_.get(), nullptr,
-                 fp32 ? geo32_.get() : geo64_.get(), lambda_, xg, sloc, done, stream_, fp32 ? tile32_ : tile64_};
+                 fp32 ? geo32_.get() : geo64_.get(), lambda_, xg, sloc, done, stream_, fp32 ? tile32_ : tile64_,
+                 edot_.as<double>()};
     NMF_HIP(launch_hex_solver(nm_, nq_, a));
 }
 
@@ -250,7 +252,8 @@ void HexSolver::autotune(int *tile64, int *tile32, std::vector<double> *times64,
         NMF_HIP(hipMemsetAsync(xg, 0x3F, NG_ * (fp32 ? sizeof(float) : sizeof(double)), stream_));
         void *sloc = fp32 ? sloc32_.get() : sloc64_.get();
         SolverArgs a{SolverKernel::Apply, fp32, deformed_, n_, N_, fp32 ? tab32_.get() : tab64_.get(), nullptr,
-                     fp32 ? geo32_.get() : geo64_.get(), lambda_, xg, sloc, nullptr, stream_, 0};
+                     fp32 ? geo32_.get() : geo64_.get(), lambda_, xg, sloc, nullptr, stream_, 0,
+                     edot_.as<double>()};
         const int best = time_tiles(
             stream_, cand,
             [&](int t) {
@@ -288,37 +291,25 @@ std::mutex &graph_capture_mutex()
     return m;
 }
 
-void HexSolver::capture_iterations(bool fp32)
+void HexSolver::capture_iterations()
 {
-    const int slot = fp32 ? 1 : 0;
-    if (graph_[slot]) return;
+    if (graph_[0]) return;
     std::lock_guard<std::mutex> lock(graph_capture_mutex());
     CGState *st = state_.as<CGState>();
     const int *done = &st->done;
+    double *x = cg64_[0].as<double>(), *r = cg64_[1].as<double>(), *p = cg64_[2].as<double>(),
+           *q = cg64_[3].as<double>(), *w = cg64_[4].as<double>();
     hipGraph_t g;
     NMF_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     for (int it = 0; it < kItersPerGraph; ++it) {
-        if (fp32) {
-            float *x = cg32_[0].as<float>(), *r = cg32_[1].as<float>(), *p = cg32_[2].as<float>(),
-                  *q = cg32_[3].as<float>(), *w = cg32_[4].as<float>(), *s = cg32_[5].as<float>();
-            NMF_HIP(solver::launch_cg_update<float>(stream_, N_, st, p, q, x, r, w, s, invd_.as<double>(),
-                                                    pa_.as<double>()));
-            apply_local(true, w, sloc32_.get(), done);
-            NMF_HIP(solver::launch_assemble<float>(stream_, n_, nm_, N_, sloc32_.as<float>(), s, w, pmu_.as<double>(),
-                                                   done));
-        } else {
-            double *x = cg64_[0].as<double>(), *r = cg64_[1].as<double>(), *p = cg64_[2].as<double>(),
-                   *q = cg64_[3].as<double>(), *w = cg64_[4].as<double>(), *s = cg64_[5].as<double>();
-            NMF_HIP(solver::launch_cg_update<double>(stream_, N_, st, p, q, x, r, w, s, invd_.as<double>(),
-                                                     pa_.as<double>()));
-            apply_local(false, w, sloc64_.get(), done);
-            NMF_HIP(solver::launch_assemble<double>(stream_, n_, nm_, N_, sloc64_.as<double>(), s, w,
-                                                    pmu_.as<double>(), done));
-        }
-        NMF_HIP(solver::launch_cg_scalar(stream_, st, pa_.as<double>(), pmu_.as<double>(), nb_));
+        NMF_HIP(solver::launch_cg_step(stream_, n_, nm_, N_, st, sloc64_.as<double>(), p, q, x, r, w,
+                                       invd_.as<double>(), pa_.as<double>()));
+        apply_local(false, w, sloc64_.get(), done);
+        NMF_HIP(solver::launch_cg_scalar(stream_, st, pa_.as<double>(), solver::cg_step_blocks(N_),
+                                         edot_.as<double>(), nelmt_));
     }
     NMF_HIP(hipStreamEndCapture(stream_, &g));
-    hipError_t e = hipGraphInstantiate(&graph_[slot], g, nullptr, nullptr, 0);
+    hipError_t e = hipGraphInstantiate(&graph_[0], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     NMF_REQUIRE(e == hipSuccess, NMF_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
 }
@@ -400,14 +391,12 @@ void HexSolver::begin_solve_enqueue(bool mixed, double tol, int maxit)
         *host_state_ = init;
         NMF_HIP(hipMemcpyAsync(state_.get(), host_state_, sizeof(CGState), hipMemcpyHostToDevice, stream_));
         double *x = cg64_[0].as<double>(), *r = cg64_[1].as<double>(), *p = cg64_[2].as<double>(),
-               *q = cg64_[3].as<double>(), *w = cg64_[4].as<double>(), *s = cg64_[5].as<double>();
+               *q = cg64_[3].as<double>(), *w = cg64_[4].as<double>();
         NMF_HIP(solver::launch_cg_init<double>(stream_, N_, b_.as<double>(), invd_.as<double>(), x, r, p, q, w,
                                                pa_.as<double>()));
         apply_local(false, w, sloc64_.get(), nullptr);
-        NMF_HIP(solver::launch_assemble<double>(stream_, n_, nm_, N_, sloc64_.as<double>(), s, w, pmu_.as<double>(),
-                                                nullptr));
-        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, pa_.as<double>(), pmu_.as<double>(), nb_));
-        capture_iterations(false);
+        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, pa_.as<double>(), nb_, edot_.as<double>(), nelmt_));
+        capture_iterations();
         job_.max_rounds = maxit / kItersPerGraph + 3;
     } else {
         ensure_fp32();

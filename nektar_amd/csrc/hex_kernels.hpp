@@ -116,6 +116,25 @@ struct StructuredFetch {
     {
         return g[((size_t)(bz + off(r)) * N + (by + off(q))) * N + (bx + off(p))];
     }
+    // line (q, r): NM consecutive nodes, vertex, bubbles, vertex, with
+    // 16-byte loads (the line starts on a value boundary only)
+    __device__ __forceinline__ void line(int q, int r, T (&x)[NM]) const
+    {
+        constexpr int VW = 16 / sizeof(T);
+        using V = T __attribute__((ext_vector_type(VW), aligned(sizeof(T))));
+        const T *l = g + ((size_t)(bz + off(r)) * N + (by + off(q))) * N + bx;
+        T v[NM];
+#pragma unroll
+        for (int c = 0; c < NM / VW; ++c) {
+            const V w = *reinterpret_cast<const V *>(l + c * VW);
+#pragma unroll
+            for (int k = 0; k < VW; ++k) v[c * VW + k] = w[k];
+        }
+#pragma unroll
+        for (int p = (NM / VW) * VW; p < NM; ++p) v[p] = l[p];
+#pragma unroll
+        for (int p = 0; p < NM; ++p) x[p] = v[off(p)];
+    }
 };
 
 // Coefficient fetch through a signed local-to-global map (GlobalToLocal
@@ -162,6 +181,8 @@ template <typename T, int NM>
 struct HasLine<LocalFetch<T, NM>> : std::true_type {};
 template <typename T, int NM>
 struct HasLine<MappedFetch<T, NM>> : std::true_type {};
+template <typename T, int NM>
+struct HasLine<StructuredFetch<T, NM>> : std::true_type {};
 
 // LDS row pitch of an element's coefficients staged as NM*NM rows (r,q)
 // of NM values: odd, so that lanes reading one row each (lane stride one
@@ -724,26 +745,53 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_grouped_kernel(int co
 }
 
 // Solver form: x gathered from the global vector of the structured n^3
-// mesh, element results written element-major (assembled afterwards).
+// mesh, element results written element-major (assembled afterwards); FP64:
+// edot[e] = x_e . y_e, its lines' sums added in the order of their indices.
 template <typename T, int NM, int NQ, int EPB>
 __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_gather_kernel(int n, int N, const T *__restrict__ tabp,
                                                                          const T *__restrict__ geo, T lambda,
                                                                          const T *__restrict__ xg,
                                                                          T *__restrict__ out,
-                                                                         const int *__restrict__ done)
+                                                                         const int *__restrict__ done,
+                                                                         double *__restrict__ edot)
 {
     if (done && *done) return;
     constexpr int TPE = NQ * NQ;
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
-    const int e = blockIdx.x * EPB + le;
     const int nelmt = n * n * n;
+    const int e = xcd_work(blockIdx.x, (nelmt + EPB - 1) / EPB) * EPB + le;
     const bool valid = e < nelmt;
     const int ex = e % n, ey = (e / n) % n, ez = e / (n * n);
     const StructuredFetch<T, NM> f{xg, N, ex * (NM - 1), ey * (NM - 1), ez * (NM - 1)};
     helmholtz_element<T, NM, NQ, true>(tab, f, valid, e, t, geo, lambda, lds[le][0], lds[le][1],
                                       out + (size_t)e * NM * NM * NM);
+    if constexpr (sizeof(T) == 8) {
+        // the staged results are still in slab 1; slab 0 is free
+        T *A = lds[le][0], *y = lds[le][1];
+        if (t < NM * NM) {
+            T s = T(0);
+#pragma unroll
+            for (int p = 0; p < NM; ++p)
+                s = fma(valid ? f(p, t % NM, t / NM) : T(0), y[t * cpitch<NM>() + p], s);
+            A[t] = s;
+        }
+        __syncthreads();
+        if (t < NM) {
+            T s = T(0);
+#pragma unroll
+            for (int r = 0; r < NM; ++r) s += A[r * NM + t];
+            A[NM * NM + t] = s;
+        }
+        __syncthreads();
+        if (t == 0 && valid) {
+            T s = T(0);
+#pragma unroll
+            for (int q = 0; q < NM; ++q) s += A[NM * NM + q];
+            edot[e] = s;
+        }
+    }
 }
 
 }  // namespace hex

@@ -116,10 +116,11 @@ template <typename T, int NM>
 constexpr bool kStaged = sizeof(T) == 8 && NM >= 9;
 
 // One element: work-item t of NM*NM, L its three slabs, g its 7 geometry
-// values {J m_00, 01, 02, 11, 12, 22, J}.
-template <typename T, int NM, int NQ, typename Fetch>
+// values {J m_00, 01, 02, 11, 12, 22, J}.  DOT: *edot = x . y of the element,
+// its lines' sums added in the order of their indices.
+template <typename T, int NM, int NQ, bool DOT = false, typename Fetch>
 __device__ __forceinline__ void element(const Fetch &fetch, bool valid, int t, const T *__restrict__ g, T lambda,
-                                        T *L, T *__restrict__ xout)
+                                        T *L, T *__restrict__ xout, double *__restrict__ edot = nullptr)
 {
     using S = Strides<T, NM>;
     constexpr int Q = S::Q, R = S::R, SL = S::SLAB;
@@ -127,8 +128,10 @@ __device__ __forceinline__ void element(const Fetch &fetch, bool valid, int t, c
     T *row = L + b * R + a * Q;  // line along direction 0: (q, r) = (a, b)
     T *mid = L + b * R + a;      // along direction 1: (n0, r) = (a, b)
     T *col = L + b * Q + a;      // along direction 2: (n0, n1) = (a, b)
+    T xl[NM];  // this work-item's line of the input
     {
-        T x[NM], u[NM], d[NM];
+        T(&x)[NM] = xl;
+        T u[NM], d[NM];
         if constexpr (hex::HasLine<Fetch>::value) {
             if (valid) {
                 fetch.line(a, b, x);
@@ -224,20 +227,41 @@ __device__ __forceinline__ void element(const Fetch &fetch, bool valid, int t, c
 #pragma unroll
         for (int p = 0; p < NM; ++p) w[p] = row[SL + p];
         transposed<NM, NQ, true>(v, w, y);
-        if constexpr (!kStaged<T, NM>) {
-            if (valid) {
+        if constexpr (DOT) {
+            double s = 0.0;
 #pragma unroll
-                for (int p = 0; p < NM; ++p) xout[t * NM + p] = y[p];
-            }
-            return;
+            for (int p = 0; p < NM; ++p) s = fma((double)xl[p], (double)y[p], s);
+            row[SL] = T(s);
         }
+        if constexpr (kStaged<T, NM>) {
 #pragma unroll
-        for (int p = 0; p < NM; ++p) row[p] = y[p];
+            for (int p = 0; p < NM; ++p) row[p] = y[p];
+        } else if (valid) {
+#pragma unroll
+            for (int p = 0; p < NM; ++p) xout[t * NM + p] = y[p];
+        }
     }
-    __syncthreads();
-    if (valid) {
+    if constexpr (kStaged<T, NM> || DOT) __syncthreads();
+    if constexpr (kStaged<T, NM>) {
+        if (valid) {
 #pragma unroll
-        for (int r = 0; r < NM; ++r) xout[r * NM * NM + t] = col[r * R];
+            for (int r = 0; r < NM; ++r) xout[r * NM * NM + t] = col[r * R];
+        }
+    }
+    if constexpr (DOT) {
+        if (t < NM) {
+            double s = 0.0;
+#pragma unroll
+            for (int r = 0; r < NM; ++r) s += (double)L[SL + r * R + t * Q];
+            L[SL + t * Q] = T(s);
+        }
+        __syncthreads();
+        if (t == 0 && valid) {
+            double s = 0.0;
+#pragma unroll
+            for (int q = 0; q < NM; ++q) s += (double)L[SL + q * Q];
+            *edot = s;
+        }
     }
 }
 
@@ -298,22 +322,27 @@ __global__ __launch_bounds__(E * NM * NM) void helmholtz_grouped_kernel(int coun
 }
 
 // Structured solver form: coefficients gathered from the global C0 vector
-// of the n^3 box
+// of the n^3 box; FP64: edot[e] = x_e . y_e, whose sum is the CG's s . w
 template <typename T, int NM, int NQ, int E>
 __global__ __launch_bounds__(E * NM * NM) void helmholtz_gather_kernel(int n, int N, const T *__restrict__ geo,
                                                                        T lambda, const T *__restrict__ xg,
                                                                        T *__restrict__ out,
-                                                                       const int *__restrict__ done)
+                                                                       const int *__restrict__ done,
+                                                                       double *__restrict__ edot)
 {
     if (done && *done) return;
     constexpr int TPE = NM * NM, NC = NM * NM * NM;
     __shared__ T lds[E][3 * Strides<T, NM>::SLAB];
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
-    const int e = blockIdx.x * E + le;
-    const bool valid = e < n * n * n;
+    const int nelmt = n * n * n;
+    const int e = xcd_work(blockIdx.x, (nelmt + E - 1) / E) * E + le;
+    const bool valid = e < nelmt;
     const int ex = e % n, ey = (e / n) % n, ez = e / (n * n);
     const hex::StructuredFetch<T, NM> f{xg, N, ex * (NM - 1), ey * (NM - 1), ez * (NM - 1)};
-    element<T, NM, NQ>(f, valid, t, geo + (size_t)e * 7, lambda, lds[le], out + (size_t)e * NC);
+    if constexpr (sizeof(T) == 8)
+        element<T, NM, NQ, true>(f, valid, t, geo + (size_t)e * 7, lambda, lds[le], out + (size_t)e * NC, edot + e);
+    else
+        element<T, NM, NQ>(f, valid, t, geo + (size_t)e * 7, lambda, lds[le], out + (size_t)e * NC);
 }
 
 }  // namespace hexmodal

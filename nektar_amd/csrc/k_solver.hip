@@ -4,9 +4,10 @@
 // N = n*(nm-1)+1), Dirichlet rows included and kept at zero, so the
 // local->global map is pure index arithmetic and never stored.
 //
-// CG (NekLinSysIterCG.cpp:118-372): every iteration is four launches -
-// update (p, q, x, r, w and the partial dots r.w, r.r), gathered operator
-// apply, assembly (with the partial dot s.w) and a one-block scalar step that
+// CG (NekLinSysIterCG.cpp:118-372): every iteration is three launches - a
+// step over the grid lines that assembles s from the element results and
+// updates p, q, x, r, w (with the partial dots r.w, r.r), the gathered operator
+// apply (with s.w as one dot per element) and a one-block scalar step that
 // finishes the reductions in a fixed order, tests ||r||^2 < tol^2 ||b||^2 and
 // forms beta and alpha.  All state (alpha, beta, rho, ..., iteration count,
 // done flag) lives in device memory, so a fixed batch of iterations can be
@@ -488,27 +489,128 @@ __global__ void cg_init_kernel(int N, const double *__restrict__ b, const double
 }
 
 // NekLinSysIterCG.cpp:240-249 (search directions, solution, residual) and
-// :264-307 (preconditioner, r.w, r.r).
-template <typename T>
-__global__ void cg_update_kernel(size_t NG, const CGState *__restrict__ st, T *__restrict__ p, T *__restrict__ q,
-                                 T *__restrict__ x, T *__restrict__ r, T *__restrict__ w, const T *__restrict__ s,
+// :264-307 (preconditioner, r.w, r.r) of one row.  The old w is M^{-1} of the
+// old r, the product that the previous step stored, so it is not read.
+struct CGRow {
+    double p, q, x, r, w;
+};
+__device__ __forceinline__ CGRow cg_row(double alpha, double beta, double p, double q, double x, double r, double s,
+                                        double inv_diag)
+{
+    CGRow o;
+    o.p = beta * p + inv_diag * r;
+    o.q = beta * q + s;
+    o.x = alpha * o.p + x;
+    o.r = -alpha * o.q + r;
+    o.w = inv_diag * o.r;
+    return o;
+}
+
+__global__ void cg_update_kernel(size_t NG, const CGState *__restrict__ st, double *__restrict__ p,
+                                 double *__restrict__ q, double *__restrict__ x, double *__restrict__ r,
+                                 double *__restrict__ w, const double *__restrict__ s,
                                  const double *__restrict__ inv_diag, double *__restrict__ partials)
 {
     if (st->done) return;
-    const T alpha = T(st->alpha), beta = T(st->beta);
+    const double alpha = st->alpha, beta = st->beta;
     double acc[2] = {0.0, 0.0};
     for (size_t G = blockIdx.x * (size_t)blockDim.x + threadIdx.x; G < NG; G += (size_t)gridDim.x * blockDim.x) {
-        const T pv = beta * p[G] + w[G];
-        const T qv = beta * q[G] + s[G];
-        x[G] = alpha * pv + x[G];
-        const T rv = -alpha * qv + r[G];
-        const T wv = T(inv_diag[G] * (double)rv);
-        p[G] = pv;
-        q[G] = qv;
-        r[G] = rv;
-        w[G] = wv;
-        acc[0] += (double)rv * (double)wv;
-        acc[1] += (double)rv * (double)rv;
+        const CGRow o = cg_row(alpha, beta, p[G], q[G], x[G], r[G], s[G], inv_diag[G]);
+        x[G] = o.x;
+        p[G] = o.p;
+        q[G] = o.q;
+        r[G] = o.r;
+        w[G] = o.w;
+        acc[0] += o.r * o.w;
+        acc[1] += o.r * o.r;
+    }
+    block_sum<2>(acc, partials + 2 * blockIdx.x);
+}
+
+// The structured solver's step: s = Assemble(sloc) as in assemble_kernel (one
+// wave per grid line, at most 8 contributions per row in a fixed order), used
+// where it is formed instead of passing through memory.  Bound by memory: 10
+// vectors and sloc per iteration, where assembly and update apart moved 15 and
+// sloc (16^3 elements at NM = 7: 9.6 + 16.7 us, this 17.7; with the lines dealt
+// out over the XCDs one by one 19.0).
+template <int NM>
+__global__ __launch_bounds__(kBlock) void cg_step_kernel(int n, int N, const CGState *__restrict__ st,
+                                                         const double *__restrict__ sloc, double *__restrict__ p,
+                                                         double *__restrict__ q, double *__restrict__ x,
+                                                         double *__restrict__ r, double *__restrict__ w,
+                                                         const double *__restrict__ inv_diag,
+                                                         double *__restrict__ partials)
+{
+    if (st->done) return;
+    const double alpha = st->alpha, beta = st->beta;
+    constexpr int WAVES = kBlock / 64, CH = 2;
+    constexpr size_t NC = (size_t)NM * NM * NM;
+    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const long lines = (long)N * N;
+    double acc[2] = {0.0, 0.0};
+    // neighbouring lines read neighbouring 8 NM byte rows of the element
+    // results: one contiguous part of the lines per XCD (gridDim: whole XCDs)
+    const int blk = xcd_work(blockIdx.x, gridDim.x);
+    for (long L = (long)blk * WAVES + wave; L < lines; L += (long)gridDim.x * WAVES) {
+        const int gz = (int)(L / N), gy = (int)(L - (long)gz * N);
+        // boundary rows hold zeros in every vector
+        if (gy == 0 || gz == 0 || gy == N - 1 || gz == N - 1) continue;
+        int ey[2], py[2], ez[2], pz[2];
+        const int cy = node_contrib<NM>(gy, n, ey, py), cz = node_contrib<NM>(gz, n, ez, pz);
+        size_t base[4] = {0, 0, 0, 0};
+        int nrow = 0;
+        for (int c = 0; c < cz; ++c)
+            for (int b = 0; b < cy; ++b)
+                base[nrow++] = ((size_t)ez[c] * n + ey[b]) * n * NC + ((size_t)pz[c] * NM + py[b]) * NM;
+        const size_t L0 = (size_t)L * N;
+        for (int gx0 = lane; gx0 < N; gx0 += 64 * CH) {
+            double v[CH][4][2], pv[CH], qv[CH], xv[CH], rv[CH], dv[CH];
+            bool live[CH];
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                const int gx = gx0 + 64 * h;
+                live[h] = gx > 0 && gx < N - 1;
+                int ex[2] = {0, 0}, px[2] = {0, 0};
+                const int cx = live[h] ? node_contrib<NM>(gx, n, ex, px) : 0;
+                const int o0 = ex[0] * (int)NC + px[0], o1 = ex[1] * (int)NC + px[1];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    v[h][k][0] = v[h][k][1] = 0.0;
+                    if (k < nrow) {  // wave-uniform
+                        const double *row = sloc + base[k];
+                        if (cx > 0) v[h][k][0] = row[o0];
+                        if (cx > 1) v[h][k][1] = row[o1];
+                    }
+                }
+                if (live[h]) {
+                    const size_t G = L0 + gx;
+                    pv[h] = p[G];
+                    qv[h] = q[G];
+                    xv[h] = x[G];
+                    rv[h] = r[G];
+                    dv[h] = inv_diag[G];
+                }
+            }
+#pragma unroll
+            for (int h = 0; h < CH; ++h) {
+                if (!live[h]) continue;
+                double s = 0.0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    s += v[h][k][0];
+                    s += v[h][k][1];
+                }
+                const CGRow o = cg_row(alpha, beta, pv[h], qv[h], xv[h], rv[h], s, dv[h]);
+                const size_t G = L0 + gx0 + 64 * h;
+                x[G] = o.x;
+                p[G] = o.p;
+                q[G] = o.q;
+                r[G] = o.r;
+                w[G] = o.w;
+                acc[0] += o.r * o.w;
+                acc[1] += o.r * o.r;
+            }
+        }
     }
     block_sum<2>(acc, partials + 2 * blockIdx.x);
 }
@@ -521,18 +623,52 @@ __device__ __forceinline__ void reduce_partials(const double *__restrict__ pa, i
     block_sum<1>(v, out);
 }
 
-__global__ void cg_scalar_init_kernel(CGState *st, const double *__restrict__ pa, const double *__restrict__ pmu,
-                                      int nb)
+// The scalar steps' reductions: A components of nb partials and the nmu
+// partials of s.w, all at once by one large block (three passes of 256
+// work-items one after another took 7.2 us, this 4.6); fixed order.
+constexpr int kScalarBlock = 1024;
+template <int A>
+__device__ __forceinline__ void reduce_scalars(const double *__restrict__ pa, int nb, const double *__restrict__ pmu,
+                                               int nmu, double (&out)[A + 1])
 {
-    __shared__ double res[4];
-    reduce_partials(pa, 3, 0, nb, &res[0]);
+    constexpr int NW = kScalarBlock / 64;
+    __shared__ double red[A + 1][NW];
+    double v[A + 1] = {};
+    for (int b = threadIdx.x; b < nb; b += kScalarBlock) {
+#pragma unroll
+        for (int c = 0; c < A; ++c) v[c] += pa[(size_t)b * A + c];
+    }
+    // four loads at a time: nmu can be one per element
+    int b = threadIdx.x;
+    for (; b + 3 * kScalarBlock < nmu; b += 4 * kScalarBlock) {
+        const double m0 = pmu[b], m1 = pmu[b + kScalarBlock], m2 = pmu[b + 2 * kScalarBlock],
+                     m3 = pmu[b + 3 * kScalarBlock];
+        v[A] += (m0 + m1) + (m2 + m3);
+    }
+    for (; b < nmu; b += kScalarBlock) v[A] += pmu[b];
+#pragma unroll
+    for (int c = 0; c <= A; ++c) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[c] += __shfl_xor(v[c], o, 64);
+        if (threadIdx.x % 64 == 0) red[c][threadIdx.x / 64] = v[c];
+    }
     __syncthreads();
-    reduce_partials(pa, 3, 1, nb, &res[1]);
-    __syncthreads();
-    reduce_partials(pa, 3, 2, nb, &res[2]);
-    __syncthreads();
-    reduce_partials(pmu, 1, 0, nb, &res[3]);
-    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    static_assert(NW == 16, "the last step adds 16 waves' sums");
+#pragma unroll
+    for (int c = 0; c <= A; ++c) {
+        double s = red[c][threadIdx.x % NW];
+#pragma unroll
+        for (int o = NW / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        out[c] = s;
+    }
+}
+
+__global__ __launch_bounds__(kScalarBlock) void cg_scalar_init_kernel(CGState *st, const double *__restrict__ pa,
+                                                                      int nb, const double *__restrict__ pmu, int nmu)
+{
+    double res[4];
+    reduce_scalars<3>(pa, nb, pmu, nmu, res);
     if (threadIdx.x != 0) return;
     const double eps = res[0], rho = res[1], bb = res[2], mu = res[3];
     st->rhs_mag = st->rhs_mag_override > 0.0 ? st->rhs_mag_override : (bb > 1.0e-6 ? bb : 1.0);  // NekLinSysIter.cpp:116
@@ -553,16 +689,12 @@ __global__ void cg_scalar_init_kernel(CGState *st, const double *__restrict__ pa
     st->iter = 1;
 }
 
-__global__ void cg_scalar_kernel(CGState *st, const double *__restrict__ pa, const double *__restrict__ pmu, int nb)
+__global__ __launch_bounds__(kScalarBlock) void cg_scalar_kernel(CGState *st, const double *__restrict__ pa, int nb,
+                                                                 const double *__restrict__ pmu, int nmu)
 {
     if (st->done) return;
-    __shared__ double res[3];
-    reduce_partials(pa, 2, 0, nb, &res[0]);
-    __syncthreads();
-    reduce_partials(pa, 2, 1, nb, &res[1]);
-    __syncthreads();
-    reduce_partials(pmu, 1, 0, nb, &res[2]);
-    __syncthreads();
+    double res[3];
+    reduce_scalars<2>(pa, nb, pmu, nmu, res);
     if (threadIdx.x != 0) return;
     const double rho_new = res[0], eps = res[1], mu = res[2];
     st->iter += 1;
@@ -922,24 +1054,41 @@ hipError_t launch_cg_init(hipStream_t stream, int N, const double *b, const doub
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_cg_update(hipStream_t stream, int N, const CGState *st, T *p, T *q, T *x, T *r, T *w, const T *s,
-                            const double *inv_diag, double *partials)
+// As many lines for every wave: a fixed grid of 8192 waves would take two
+// rounds over the 9,409 lines of 16^3 elements at NM = 7, the second nearly
+// empty (measured: no difference).
+int cg_step_blocks(int N)
 {
-    const size_t NG = (size_t)N * N * N;
-    NMF_LAUNCH((cg_update_kernel<T>), grid_for(NG), NG, st, p, q, x, r, w, s, inv_diag, partials);
+    const long waves = kBlock / 64, lines = (long)N * N;
+    static_assert(kRedBlocks % kXcds == 0, "the partials hold whole XCDs' blocks");
+    const long per = (lines + waves * kRedBlocks - 1) / (waves * kRedBlocks);
+    return xcd_grid((int)((lines + waves * per - 1) / (waves * per)));
+}
+
+hipError_t launch_cg_step(hipStream_t stream, int n, int nm, int N, const CGState *st, const double *sloc, double *p,
+                          double *q, double *x, double *r, double *w, const double *inv_diag, double *partials)
+{
+    const int grid = cg_step_blocks(N);
+    switch (nm) {
+#define NMF_STEP(M) \
+    case M: NMF_LAUNCH((cg_step_kernel<M>), grid, n, N, st, sloc, p, q, x, r, w, inv_diag, partials); break;
+        NMF_STEP(2) NMF_STEP(3) NMF_STEP(4) NMF_STEP(5) NMF_STEP(6) NMF_STEP(7) NMF_STEP(8) NMF_STEP(9) NMF_STEP(10)
+#undef NMF_STEP
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_cg_scalar_init(hipStream_t stream, CGState *st, const double *pa, const double *pmu, int nb)
+hipError_t launch_cg_scalar_init(hipStream_t stream, CGState *st, const double *pa, int nb, const double *pmu,
+                                 int nmu)
 {
-    NMF_LAUNCH(cg_scalar_init_kernel, 1, st, pa, pmu, nb);
+    hipLaunchKernelGGL(cg_scalar_init_kernel, dim3(1), dim3(kScalarBlock), 0, stream, st, pa, nb, pmu, nmu);
     return hipGetLastError();
 }
 
-hipError_t launch_cg_scalar(hipStream_t stream, CGState *st, const double *pa, const double *pmu, int nb)
+hipError_t launch_cg_scalar(hipStream_t stream, CGState *st, const double *pa, int nb, const double *pmu, int nmu)
 {
-    NMF_LAUNCH(cg_scalar_kernel, 1, st, pa, pmu, nb);
+    hipLaunchKernelGGL(cg_scalar_kernel, dim3(1), dim3(kScalarBlock), 0, stream, st, pa, nb, pmu, nmu);
     return hipGetLastError();
 }
 
@@ -1093,8 +1242,6 @@ template hipError_t launch_assemble<float>(hipStream_t, int, int, int, const flo
                                            const int *, bool);
 template hipError_t launch_cg_init<double>(hipStream_t, int, const double *, const double *, double *, double *,
                                            double *, double *, double *, double *);
-template hipError_t launch_cg_init<float>(hipStream_t, int, const double *, const double *, float *, float *, float *,
-                                          float *, float *, double *);
 hipError_t launch_gather_signed(hipStream_t stream, size_t nloc, const int *menc, const double *glob, double *loc)
 {
     NMF_LAUNCH(gather_signed_kernel, grid_for(nloc), nloc, menc, glob, loc);
@@ -1138,7 +1285,7 @@ hipError_t launch_cg_init_dirfirst(hipStream_t stream, int nglob, int ndir, cons
 hipError_t launch_cg_update_n(hipStream_t stream, size_t NG, const CGState *st, double *p, double *q, double *x,
                               double *r, double *w, const double *s, const double *inv_diag, double *partials)
 {
-    NMF_LAUNCH((cg_update_kernel<double>), grid_for(NG), NG, st, p, q, x, r, w, s, inv_diag, partials);
+    NMF_LAUNCH(cg_update_kernel, grid_for(NG), NG, st, p, q, x, r, w, s, inv_diag, partials);
     return hipGetLastError();
 }
 
@@ -1181,10 +1328,6 @@ hipError_t launch_csr_first(hipStream_t stream, int nglob, const int *row, const
     return hipGetLastError();
 }
 
-template hipError_t launch_cg_update<double>(hipStream_t, int, const CGState *, double *, double *, double *, double *,
-                                             double *, const double *, const double *, double *);
-template hipError_t launch_cg_update<float>(hipStream_t, int, const CGState *, float *, float *, float *, float *,
-                                            float *, const float *, const double *, double *);
 template hipError_t launch_add<float>(hipStream_t, size_t, double *, const float *);
 template hipError_t launch_add<double>(hipStream_t, size_t, double *, const double *);
 

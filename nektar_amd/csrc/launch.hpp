@@ -51,6 +51,7 @@ struct SolverArgs {
     const int *done;   // Apply: early exit flag (NULL = always run)
     hipStream_t stream;
     int tile = 0;      // Apply: elements per workgroup (0 = default)
+    double *edot = nullptr;  // FP64 Apply: in_e . out_e per element (required)
 };
 
 // Tile shapes (elements per workgroup) available for the hex Helmholtz
@@ -80,6 +81,18 @@ struct GroupArgs {
     hipStream_t stream;
     int tile = 0;       // hex: elements per workgroup (0 = default)
 };
+
+// Workgroups go to the 8 XCDs in turn, and each XCD has an L2 of its own.
+// Kernels whose neighbouring workgroups share cache lines (solver forms: the
+// nodes of neighbouring elements, the rows of one) give every XCD one
+// contiguous part: work b of n on a grid of xcd_grid(n) workgroups (the last
+// ones have none: >= n).
+constexpr int kXcds = 8;
+constexpr int xcd_grid(int n) { return (n + kXcds - 1) / kXcds * kXcds; }
+__host__ __device__ inline int xcd_work(int block, int n)
+{
+    return (block % kXcds) * ((n + kXcds - 1) / kXcds) + block / kXcds;
+}
 
 // Elements per workgroup: hex default fill (tile 0) or the given tile.
 // A tet tile is the number of work-items per element: packed

@@ -51,11 +51,13 @@ hipError_t launch_assemble(hipStream_t, int n, int nm, int N, const T *sloc, T *
 template <typename T>
 hipError_t launch_cg_init(hipStream_t, int N, const double *b, const double *inv_diag, T *x, T *r, T *p, T *q, T *w,
                           double *partials);
-template <typename T>
-hipError_t launch_cg_update(hipStream_t, int N, const CGState *st, T *p, T *q, T *x, T *r, T *w, const T *s,
-                            const double *inv_diag, double *partials);
-hipError_t launch_cg_scalar_init(hipStream_t, CGState *st, const double *pa, const double *pmu, int nb);
-hipError_t launch_cg_scalar(hipStream_t, CGState *st, const double *pa, const double *pmu, int nb);
+// assembly of the element results and the CG's vector updates in one pass
+hipError_t launch_cg_step(hipStream_t, int n, int nm, int N, const CGState *st, const double *sloc, double *p,
+                          double *q, double *x, double *r, double *w, const double *inv_diag, double *partials);
+int cg_step_blocks(int N);  // its partials
+// nb partials of the vector dots, nmu of s.w
+hipError_t launch_cg_scalar_init(hipStream_t, CGState *st, const double *pa, int nb, const double *pmu, int nmu);
+hipError_t launch_cg_scalar(hipStream_t, CGState *st, const double *pa, int nb, const double *pmu, int nmu);
 hipError_t launch_residual(hipStream_t, int N, const double *b, const double *s, double *r, double *partials);
 // Hestenes-Stiefel PCG (used for the FP32 inner solve of the mixed path)
 template <typename T>
@@ -203,7 +205,7 @@ private:
     void build_diagonal();
     void apply_local(bool fp32, const void *xg, void *sloc, const int *done);
     void apply_global_fp64(const double *x, double *y);  // no state check (used inside solves)
-    void capture_iterations(bool fp32);
+    void capture_iterations();
     void assemble_rhs(const double *f_dev);
     void enqueue_state_read();
     void enqueue_reliable_update();
@@ -233,8 +235,9 @@ private:
     DeviceBuffer b_, x_, invd_, sloc64_, tmp64_, r64_;
     DeviceBuffer invd32_;  // FP32 copy of invd_ for the FP32 iterations of the mixed solve
     // CG work vectors per precision
-    DeviceBuffer cg64_[6], cg32_[6], sloc32_;  // x r p q w s
+    DeviceBuffer cg64_[5], cg32_[6], sloc32_;  // x r p q w (s)
     DeviceBuffer state_, pa_, pmu_, scalar_;
+    DeviceBuffer edot_;  // w_e . (A w)_e per element
     solver::CGState *host_state_ = nullptr;
     double *host_scalar_ = nullptr;
 

@@ -141,5 +141,24 @@ __global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void bwd_gather
     }
 }
 
+// edot[e] = x_e . y_e, x gathered from the global vector, y element-major
+// (for the gather-apply tiles that do not form it themselves)
+template <int NM>
+__global__ __launch_bounds__(64) void element_dot_kernel(int n, int N, const double *__restrict__ xg,
+                                                         const double *__restrict__ y, const int *__restrict__ done,
+                                                         double *__restrict__ edot)
+{
+    if (done && *done) return;
+    constexpr int NC = NM * NM * NM;
+    const int e = blockIdx.x, t = threadIdx.x;
+    const int ex = e % n, ey = (e / n) % n, ez = e / (n * n);
+    const StructuredFetch<double, NM> f{xg, N, ex * (NM - 1), ey * (NM - 1), ez * (NM - 1)};
+    double s = 0.0;
+    for (int m = t; m < NC; m += 64) s = fma(f(m % NM, (m / NM) % NM, m / (NM * NM)), y[(size_t)e * NC + m], s);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (t == 0) edot[e] = s;
+}
+
 }  // namespace hex
 }  // namespace nektar_amd

@@ -304,7 +304,7 @@ SolveInfo IterativeSolver::solve_static_cond(double tol, int maxit)
         NMF_HIP(solver::launch_cg_init_dirfirst(stream_, NB, ND, d.bvec.as<double>(), d.invd_b.as<double>(), x, r, p,
                                                 q, w, d.pa.as<double>()));
         matvec();
-        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, d.pa.as<double>(), d.pmu.as<double>(), d.nred));
+        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, d.pa.as<double>(), d.nred, d.pmu.as<double>(), d.nred));
         const int max_rounds = maxit / kItersPerChunk + 3;
         for (int round = 0;; ++round) {
             NMF_HIP(hipMemcpyAsync(host_state_, st, sizeof(solver::CGState), hipMemcpyDeviceToHost, stream_));
@@ -314,7 +314,7 @@ SolveInfo IterativeSolver::solve_static_cond(double tol, int maxit)
                 NMF_HIP(solver::launch_cg_update_n(stream_, (size_t)NB, st, p, q, x, r, w, s, d.invd_b.as<double>(),
                                                    d.pa.as<double>()));
                 matvec();
-                NMF_HIP(solver::launch_cg_scalar(stream_, st, d.pa.as<double>(), d.pmu.as<double>(), d.nred));
+                NMF_HIP(solver::launch_cg_scalar(stream_, st, d.pa.as<double>(), d.nred, d.pmu.as<double>(), d.nred));
             }
         }
         // V_bnd = GlobalToLocalBnd(x); V_int = A_ii^-1 (F_int - A_ib V_bnd)

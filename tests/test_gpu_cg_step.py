@@ -1,0 +1,42 @@
+"""The structured solver's CG iteration in three launches (assembly fused with
+the vector updates, s.w as one dot per element): every compiled NUMMODES,
+meshes whose grid lines do not fill the 64- and 128-row pieces of a wave or
+whose line count does not divide among the XCDs, the smallest mesh, affine and
+perturbed elements.
+
+The dots only steer the iteration, so a wrong one shows as a residual that the
+recurrence does not know of: the true residual b - A x, taken with
+apply_global (assembled by another kernel), has to be what the solve reports.
+The recurrence residual is below 1e-10 ||b||; rounding of some hundred updates
+of a system of condition below 1e6 adds less than 1e-9 ||b||."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def nmf():
+    assert torch.cuda.is_available(), "GPU tests need a GPU"
+    import nektar_amd
+    nektar_amd.lib()
+    return nektar_amd
+
+
+@pytest.mark.parametrize("nm", range(2, 11))
+@pytest.mark.parametrize("perturb", [0.0, 0.1], ids=["affine", "perturbed"])
+def test_true_residual(nmf, nm, perturb):
+    for n in (2, 3, 13 if nm == 6 else 7 if nm < 9 else 4):
+        s = nmf.HelmholtzSolver(n, nm, nm + 1, 1.3, perturb=perturb, seed=3)
+        s.set_forcing_manufactured(1)
+        info = s.solve(tol=1e-10, maxit=8000)
+        assert info.converged, (n, info.as_dict())
+        x = torch.from_numpy(s.solution()).cuda()
+        y = torch.zeros_like(x)
+        s.apply_global(x, y)
+        torch.cuda.synchronize()
+        b, N = s.rhs().reshape((n * (nm - 1) + 1,) * 3), n * (nm - 1) + 1
+        res = (b - y.cpu().numpy().reshape(b.shape))[1:N - 1, 1:N - 1, 1:N - 1]
+        assert np.linalg.norm(res) <= 1.1e-9 * np.linalg.norm(b), (n, np.linalg.norm(res) / np.linalg.norm(b))
