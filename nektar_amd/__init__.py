@@ -249,6 +249,7 @@ class Operator:
                                       ctypes.byref(de), ctypes.byref(pr)))
         self.ncoeff, self.nqtot, self.nelmt = nc.value, nq.value, ne.value
         self.deformed, self.precision = bool(de.value), pr.value
+        self._io = None
 
     def __del__(self):
         if getattr(self, "_h", None) is not None and _LIB is not None:
@@ -292,8 +293,15 @@ class Operator:
 
     # --- sizes (Collections::Operator::GetInputSize/GetOutputSize) --------
     def _io_size(self):
+        # fixed by the operator's kind and sizes, except where the scaling
+        # factor changes them: kept, so that a small apply does not wait for
+        # two more calls through ctypes (8.0 -> 6.5 us per call)
+        if self._io is not None:
+            return self._io
         a, b = ctypes.c_int64(), ctypes.c_int64()
         check(lib().nmf_operator_io_size(self._h, ctypes.byref(a), ctypes.byref(b)))
+        if self.op != "PhysInterp1DScaled":
+            self._io = (a.value, b.value)
         return a.value, b.value
 
     def input_size(self) -> int:
