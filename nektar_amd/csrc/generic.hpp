@@ -21,6 +21,7 @@ struct GenArgs {
     int nelmt;
     int nm[3], nq[3], nqtot, ncoeff;
     int npq;   // tets: (p, q) pairs, sum_p (nm1 - p)
+    int ntab, nitab;  // entries of tab and itab
     int buf;   // values per intermediate buffer (four per element)
     // offsets (in values) of the tables in `tab`: B_d [mode*nq_d + i],
     // D_d [l*nq_d + i] (= l_l'(z_i)), W_d (Radau pre-scaled), and the tet
@@ -62,5 +63,20 @@ int generic_ncoeffs(Shape s, const int nm[3]);
 void generic_check(Shape s, const int nm[3], const int nq[3]);
 GenLayout generic_layout(Shape s, const int nm[3], const int nq[3]);
 hipError_t launch_generic(const GenArgs &a);
+
+// Prisms and pyramids with compile-time sizes (gen_fixed.hpp): equal modes in
+// the three directions and the default points (Q, Q, Q - 1) with Q = NM + 1 or
+// NM + 2, NM = 3 .. 7.  Prisms, 4,096 elements, FP64 us on the runtime-size
+// kernels and here: NM = 3 26.8/7.2, 4 34.8/12.6, 5 45.5/19.9, 6 70.6/33.3,
+// 7 106/57; 50 elements at NM = 3 9.0/4.3, 7 18.0/9.0.
+constexpr int kFixedMinModes = 3, kFixedMaxModes = 7;
+inline bool fixed_sizes(const GenArgs &a)
+{
+    return (a.shape == Shape::Prism || a.shape == Shape::Pyr) && a.nm[1] == a.nm[0] && a.nm[2] == a.nm[0] &&
+           a.nm[0] >= kFixedMinModes && a.nm[0] <= kFixedMaxModes && a.nq[1] == a.nq[0] && a.nq[2] == a.nq[0] - 1 &&
+           (a.nq[0] == a.nm[0] + 1 || a.nq[0] == a.nm[0] + 2);
+}
+hipError_t launch_fixed_prism(const GenArgs &a);
+hipError_t launch_fixed_pyr(const GenArgs &a);
 
 }  // namespace nektar_amd

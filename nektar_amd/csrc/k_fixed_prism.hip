@@ -1,0 +1,8 @@
+// Prism operators with compile-time sizes.
+#include "gen_fixed.hpp"
+
+namespace nektar_amd {
+
+hipError_t launch_fixed_prism(const GenArgs &a) { return gen::launch_fixed_shape<gen::SH_PRISM>(a); }
+
+}  // namespace nektar_amd

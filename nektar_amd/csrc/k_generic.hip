@@ -69,6 +69,7 @@ hipError_t launch_t(const GenArgs &a)
 
 hipError_t launch_generic(const GenArgs &a)
 {
+    if (fixed_sizes(a)) return a.shape == Shape::Prism ? launch_fixed_prism(a) : launch_fixed_pyr(a);
     if (a.shape == Shape::Hex)
         return a.fp32 ? gen::launch_t<float, gen::SH_HEX>(a) : gen::launch_t<double, gen::SH_HEX>(a);
     if (a.shape == Shape::Prism)

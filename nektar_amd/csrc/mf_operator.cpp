@@ -183,6 +183,8 @@ GenArgs MFOperator::generic_args(const void *in0, const void *in1, const void *i
     a.nqtot = nqtot;
     a.ncoeff = ncoeff;
     a.npq = glay.npq;
+    a.ntab = (int)glay.tab.size();
+    a.nitab = (int)glay.itab.size();
     a.buf = glay.buf;
     a.tab = tab.get();
     a.itab = gitab.as<int>();
