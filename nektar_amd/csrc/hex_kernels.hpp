@@ -305,31 +305,6 @@ __device__ __forceinline__ void iprod_from_column(const Tab<T, NM, NQ> &tab, con
     }
 }
 
-// ---- collocation derivatives in directions 0 and 1 from slab A (u),
-//      written to slabs Bs (d0) and C (d1).  Direction 2 is in registers.
-template <typename T, int NM, int NQ>
-__device__ __forceinline__ void deriv01(const Tab<T, NM, NQ> &tab, int t, const T *A, T *Bs, T *C)
-{
-    constexpr int P = pitch<NQ>();
-    const int l0 = t % NQ, k = t / NQ;
-    {   // line (j = l0, k) along i
-        T v[NQ], o[NQ];
-#pragma unroll
-        for (int l = 0; l < NQ; ++l) v[l] = A[(k * NQ + l0) * P + l];
-        contract<false>(v, [&](int i) { return tab.DTrow(i); }, o);
-#pragma unroll
-        for (int i = 0; i < NQ; ++i) Bs[(k * NQ + l0) * P + i] = o[i];
-    }
-    {   // line (i = l0, k) along j
-        T v[NQ], o[NQ];
-#pragma unroll
-        for (int l = 0; l < NQ; ++l) v[l] = A[(k * NQ + l) * P + l0];
-        contract<false>(v, [&](int j) { return tab.DTrow(j); }, o);
-#pragma unroll
-        for (int j = 0; j < NQ; ++j) C[(k * NQ + j) * P + l0] = o[j];
-    }
-}
-
 template <typename T, int NM, int NQ>
 __device__ __forceinline__ void deriv2_column(const Tab<T, NM, NQ> &tab, const T (&u)[NQ], T (&d2)[NQ])
 {
@@ -338,11 +313,11 @@ __device__ __forceinline__ void deriv2_column(const Tab<T, NM, NQ> &tab, const T
 
 // ===================================================================
 // BwdTrans (BwdTransKernels.hpp:160-227)
-template <typename T, int NM, int NQ>
-__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void bwdtrans_kernel(
+template <typename T, int NM, int NQ, int EPB>
+__global__ __launch_bounds__(EPB * NQ * NQ) void bwdtrans_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ in, T *__restrict__ out)
 {
-    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
+    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
@@ -360,12 +335,12 @@ __global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void bwdtrans_k
 }
 
 // IProductWRTBase (IProductKernels.hpp:270-350, SCALE=APPEND=false)
-template <typename T, int NM, int NQ, bool DEF>
-__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void iproduct_kernel(
+template <typename T, int NM, int NQ, bool DEF, int EPB>
+__global__ __launch_bounds__(EPB * NQ * NQ) void iproduct_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ jac, const T *__restrict__ in,
     T *__restrict__ out)
 {
-    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
+    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
@@ -388,19 +363,19 @@ __global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void iproduct_k
 }
 
 // PhysDeriv (PhysDerivKernels.hpp:436-507 then :326-340)
-template <typename T, int NM, int NQ, bool DEF>
-__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void physderiv_kernel(
+template <typename T, int NM, int NQ, bool DEF, int EPB>
+__global__ __launch_bounds__(EPB * NQ * NQ) void physderiv_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ df, const T *__restrict__ in,
     T *__restrict__ out0, T *__restrict__ out1, T *__restrict__ out2)
 {
-    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
-    __shared__ T lds[EPB][3][slab<NQ>()];
+    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
+    __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
     const int e = blockIdx.x * EPB + le;
     const bool valid = e < nelmt;
     const int i = t % NQ, j = t / NQ;
-    T *A = lds[le][0], *Bs = lds[le][1], *C = lds[le][2];
+    T *A = lds[le][0], *Bs = lds[le][1];
     T u[NQ], d2[NQ];
     const T *f = in + (size_t)e * NQ3;
 #pragma unroll
@@ -411,7 +386,23 @@ __global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void physderiv_
     }
     deriv2_column<T, NM, NQ>(tab, u, d2);
     __syncthreads();
-    deriv01<T, NM, NQ>(tab, t, A, Bs, C);
+    {   // d0 along direction 0 on line (j, k) = (i, j): A -> Bs
+        T v[NQ], o[NQ];
+#pragma unroll
+        for (int l = 0; l < NQ; ++l) v[l] = A[(j * NQ + i) * pitch<NQ>() + l];
+        contract<false>(v, [&](int ii) { return tab.DTrow(ii); }, o);
+#pragma unroll
+        for (int ii = 0; ii < NQ; ++ii) Bs[(j * NQ + i) * pitch<NQ>() + ii] = o[ii];
+    }
+    __syncthreads();
+    {   // d1 along direction 1 on line (i, k) = (i, j), in place in A
+        T v[NQ], o[NQ];
+#pragma unroll
+        for (int l = 0; l < NQ; ++l) v[l] = A[(j * NQ + l) * pitch<NQ>() + i];
+        contract<false>(v, [&](int jj) { return tab.DTrow(jj); }, o);
+#pragma unroll
+        for (int jj = 0; jj < NQ; ++jj) A[(j * NQ + jj) * pitch<NQ>() + i] = o[jj];
+    }
     __syncthreads();
     if (!valid) return;
     T g[9];
@@ -427,7 +418,7 @@ __global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void physderiv_
             for (int d = 0; d < 9; ++d) g[d] = df[((size_t)e * 9 + d) * NQ3 + c];
         }
         const int lc = (k * NQ + j) * pitch<NQ>() + i;
-        const T a0 = Bs[lc], a1 = C[lc], a2 = d2[k];
+        const T a0 = Bs[lc], a1 = A[lc], a2 = d2[k];
         T o0 = a0 * g[0];
         o0 = fma(a1, g[1], o0);
         o0 = fma(a2, g[2], o0);
@@ -603,12 +594,12 @@ __device__ __forceinline__ void helmholtz_element(const Tab<T, NM, NQ> &tab, con
 // t_d) with t_d = sum_j df[j*3+d] in_j.  Packed geometry: regular
 // g[e*9 + j*3+d] = J df[j*3+d] (weights applied here); deformed
 // g[(e*9 + j*3+d)*Q^3 + q] = W_q J_q df_q[j*3+d].
-template <typename T, int NM, int NQ, bool DEF>
-__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void iproduct_deriv_kernel(
+template <typename T, int NM, int NQ, bool DEF, int EPB>
+__global__ __launch_bounds__(EPB * NQ * NQ) void iproduct_deriv_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ geo, const T *__restrict__ in0,
     const T *__restrict__ in1, const T *__restrict__ in2, T *__restrict__ out)
 {
-    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ, P = pitch<NQ>();
+    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ, P = pitch<NQ>();
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
