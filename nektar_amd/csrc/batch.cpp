@@ -145,7 +145,8 @@ void Batch::build()
         groups_[it->second].members.push_back(i);
     }
     for (auto &g : groups_) {
-        const int epb = g.shape == Shape::Hex ? hex_tile_elems(g.nm, g.nq, g.deformed, g.tile) : tet_tile_elems(g.nq, g.tile);
+        const int epb = g.shape == Shape::Hex ? hex_tile_elems(g.nm, g.nq, g.deformed, g.fp32, g.tile)
+                                              : tet_tile_elems(g.nq, g.tile);
         int block0 = 0;
         std::vector<GroupItem<double>> i64;
         std::vector<GroupItem<float>> i32;

@@ -114,11 +114,23 @@ constexpr int hex_modal_elems(int nm)
 {
     return nm <= 4 ? 64 / (nm * nm) : nm <= 6 ? 5 : nm == 9 ? 2 : 1;
 }
+// Default tile of the kernels with per-point geometry: the matrix-core tile
+// of one element where its 16-row products are well filled and the vector
+// kernel's are not bound by memory yet.  Measured vector / matrix cores, us on
+// 1.6 M points: FP64 NM, NQ = 6, 8 35.5/23.2; 7, 8 37/25; 8, 9 28/39; 8, 10
+// 41/32; 9, 10 42/37; 10, 11 47/34; 10, 12 47/38; 6, 7 27/27; 5, 7 26/26; FP32
+// 7, 8 16.8/15.8; 8, 10 21/22; 10, 11 23/19; 10, 12 25/20.
+constexpr int hex_deformed_tile(int nm, int nq, bool fp32)
+{
+    const bool mfma = nm >= 6 && (fp32 ? nq == 8 || nq >= 11 : nq == 8 || nq >= 10);
+    return mfma ? kMfmaTile + 1 : hex_fill_elems(nq);
+}
 // elements per workgroup of a tile (0: the default) of a hex Helmholtz kind
-inline int hex_tile_elems(int nm, int nq, bool deformed, int tile)
+inline int hex_tile_elems(int nm, int nq, bool deformed, bool fp32, int tile)
 {
     if (tile <= 0 && !deformed) return hex_modal_elems(nm);
-    return tile >= kMfmaTile ? tile - kMfmaTile : (tile > 0 ? tile : hex_fill_elems(nq));
+    if (tile <= 0) tile = hex_deformed_tile(nm, nq, fp32);
+    return tile >= kMfmaTile ? tile - kMfmaTile : tile;
 }
 constexpr int tet_packed_tpe(int nq0) { return nq0 * (nq0 - 1); }
 constexpr int tet_wave_tpe(int nq0) { return (nq0 * (nq0 - 1) + 63) / 64 * 64; }
