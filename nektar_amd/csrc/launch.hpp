@@ -118,8 +118,9 @@ constexpr int hex_modal_elems(int nm)
 // of one element where its 16-row products are well filled and the vector
 // kernel's are not bound by memory yet.  Measured vector / matrix cores, us on
 // 1.6 M points: FP64 NM, NQ = 6, 8 35.5/23.2; 7, 8 37/25; 8, 9 28/39; 8, 10
-// 41/32; 9, 10 42/37; 10, 11 47/34; 10, 12 47/38; 6, 7 27/27; 5, 7 26/26; FP32
-// 7, 8 16.8/15.8; 8, 10 21/22; 10, 11 23/19; 10, 12 25/20.
+// 41/32; 9, 10 42/37; 10, 11 47/34; 10, 12 47/38; 8, 8 40/26; 10, 10 44/39;
+// 6, 7 27/27; 5, 7 26/26; FP32 7, 8 16.8/15.8; 8, 8 17.5/14.8; 8, 10 21/22;
+// 10, 11 23/19; 10, 12 25/20.
 constexpr int hex_deformed_tile(int nm, int nq, bool fp32)
 {
     const bool mfma = nm >= 6 && (fp32 ? nq == 8 || nq >= 11 : nq == 8 || nq >= 10);
