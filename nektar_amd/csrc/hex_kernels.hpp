@@ -7,8 +7,9 @@
 // inputs once, keeps them in registers and produces all outputs of the line,
 // so every LDS read feeds NQ fused multiply-adds.  The 1-D tables (basis,
 // derivative matrix, weights) are wave-uniform and live in scalar registers
-// (loaded with scalar loads from the operator's table buffer).  Three LDS
-// slabs of NQ^3 values per element carry the tensor between directions.
+// (loaded with scalar loads from the operator's table buffer).  LDS
+// slabs of NQ^3 values per element (two, or three where a kernel keeps all
+// derivatives) carry the tensor between directions.
 //
 // Layouts (element-major, the Collections contract):
 //   coefficients  in[e*NM^3 + (r*NM + q)*NM + p]     (p fastest)
