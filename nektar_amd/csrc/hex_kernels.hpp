@@ -363,20 +363,22 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void iproduct_kernel(
     iprod_from_column<T, NM, NQ>(tab, y, valid, t, lds[le][0], lds[le][1], out + (size_t)e * NM * NM * NM);
 }
 
-// PhysDeriv (PhysDerivKernels.hpp:436-507 then :326-340)
-template <typename T, int NM, int NQ, bool DEF, int EPB>
-__global__ __launch_bounds__(EPB * NQ * NQ) void physderiv_kernel(
+// PhysDeriv (PhysDerivKernels.hpp:436-507 then :326-340).  With three slabs
+// the passes of directions 0 and 1 run side by side; with two the second one
+// works in place, behind a barrier of its own, and more workgroups fit a CU.
+template <typename T, int NM, int NQ, bool DEF, int SLABS>
+__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void physderiv_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ df, const T *__restrict__ in,
     T *__restrict__ out0, T *__restrict__ out1, T *__restrict__ out2)
 {
-    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
-    __shared__ T lds[EPB][2][slab<NQ>()];
+    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
+    __shared__ T lds[EPB][SLABS][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
     const int e = blockIdx.x * EPB + le;
     const bool valid = e < nelmt;
     const int i = t % NQ, j = t / NQ;
-    T *A = lds[le][0], *Bs = lds[le][1];
+    T *A = lds[le][0], *Bs = lds[le][1], *C = lds[le][SLABS == 2 ? 0 : 2];
     T u[NQ], d2[NQ];
     const T *f = in + (size_t)e * NQ3;
 #pragma unroll
@@ -395,14 +397,14 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void physderiv_kernel(
 #pragma unroll
         for (int ii = 0; ii < NQ; ++ii) Bs[(j * NQ + i) * pitch<NQ>() + ii] = o[ii];
     }
-    __syncthreads();
-    {   // d1 along direction 1 on line (i, k) = (i, j), in place in A
+    if constexpr (SLABS == 2) __syncthreads();
+    {   // d1 along direction 1 on line (i, k) = (i, j): A -> C
         T v[NQ], o[NQ];
 #pragma unroll
         for (int l = 0; l < NQ; ++l) v[l] = A[(j * NQ + l) * pitch<NQ>() + i];
         contract<false>(v, [&](int jj) { return tab.DTrow(jj); }, o);
 #pragma unroll
-        for (int jj = 0; jj < NQ; ++jj) A[(j * NQ + jj) * pitch<NQ>() + i] = o[jj];
+        for (int jj = 0; jj < NQ; ++jj) C[(j * NQ + jj) * pitch<NQ>() + i] = o[jj];
     }
     __syncthreads();
     if (!valid) return;
@@ -419,7 +421,7 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void physderiv_kernel(
             for (int d = 0; d < 9; ++d) g[d] = df[((size_t)e * 9 + d) * NQ3 + c];
         }
         const int lc = (k * NQ + j) * pitch<NQ>() + i;
-        const T a0 = Bs[lc], a1 = A[lc], a2 = d2[k];
+        const T a0 = Bs[lc], a1 = C[lc], a2 = d2[k];
         T o0 = a0 * g[0];
         o0 = fma(a1, g[1], o0);
         o0 = fma(a2, g[2], o0);
@@ -433,6 +435,29 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void physderiv_kernel(
         out1[(size_t)e * NQ3 + c] = o1;
         out2[(size_t)e * NQ3 + c] = o2;
     }
+}
+
+// Two slabs where the workgroups no longer fit the 256 CUs at once with three
+// (160 KB of LDS and 32 waves each): the smaller footprint then pays for the
+// barrier, FP64 us with three and two slabs, constant df, 1.5 M points: Q = 6
+// 13.4/11.0, 7 15.6/12.0, 8 16.4/13.1, 11 20.6/15.5, 12 20.7/15.4.  Below, the
+// barrier only costs: Q = 9, 2,057 elements 13.3/14.0, FP32 Q = 11, 1,126
+// elements 9.2/9.7.  At Q = 4 in FP64 two slabs win only while they hold at
+// once what three do not (per-point df, 23,437 elements 25/24, 93,750 elements
+// 110.7/112.7), at Q = 5 nowhere (12,000 elements 25.5/29.5, 48,000 124/141),
+// nor at Q = 3 and, in FP32, 4.
+template <typename T, int NQ>
+bool physderiv_two_slabs(int nelmt)
+{
+    if constexpr (NQ < 6 && !(NQ == 4 && sizeof(T) == 8)) return false;
+    constexpr int EPB = elements_per_block<NQ>(), WAVES = (EPB * NQ * NQ + 63) / 64;
+    constexpr int SLAB = EPB * slab<NQ>() * (int)sizeof(T);
+    const auto held = [](int slabs) {
+        const int lds = 160 * 1024 / (slabs * SLAB), waves = 32 / WAVES;
+        return 256 * (lds < waves ? lds : waves);
+    };
+    const int blocks = (nelmt + EPB - 1) / EPB;
+    return blocks > held(3) && (NQ > 4 || blocks <= held(2));
 }
 
 // Second half shared by the fused Helmholtz apply and IProductWRTDerivBase:
