@@ -129,14 +129,18 @@ void Batch::build()
             singles_.push_back(i);
             continue;
         }
-        const auto key = std::make_tuple((int)o.shape, o.nm, o.nq[0], o.tile, (int)o.fp32, (int)o.deformed);
+        // the default of curved hexes depends on the member's size
+        const int tile = o.tile == 0 && o.shape == Shape::Hex && o.deformed
+                             ? hex_deformed_tile(o.nm, o.nq[0], o.fp32, o.nelmt)
+                             : o.tile;
+        const auto key = std::make_tuple((int)o.shape, o.nm, o.nq[0], tile, (int)o.fp32, (int)o.deformed);
         auto it = index.find(key);
         if (it == index.end()) {
             Group g;
             g.shape = o.shape;
             g.nm = o.nm;
             g.nq = o.nq[0];
-            g.tile = o.tile;
+            g.tile = tile;
             g.fp32 = o.fp32;
             g.deformed = o.deformed;
             groups_.push_back(std::move(g));
@@ -145,7 +149,7 @@ void Batch::build()
         groups_[it->second].members.push_back(i);
     }
     for (auto &g : groups_) {
-        const int epb = g.shape == Shape::Hex ? hex_tile_elems(g.nm, g.nq, g.deformed, g.fp32, g.tile)
+        const int epb = g.shape == Shape::Hex ? hex_tile_elems(g.nm, g.tile)
                                               : tet_tile_elems(g.nq, g.tile);
         int block0 = 0;
         std::vector<GroupItem<double>> i64;

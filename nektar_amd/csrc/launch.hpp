@@ -79,7 +79,7 @@ struct GroupArgs {
     int nblocks;        // total workgroups of the launch
     const void *tab;    // tables shared by every item of the kind
     hipStream_t stream;
-    int tile = 0;       // hex: elements per workgroup (0 = default)
+    int tile = 0;       // hex: elements per workgroup (0 = default, affine elements only)
 };
 
 // Workgroups go to the 8 XCDs in turn, and each XCD has an L2 of its own.
@@ -120,17 +120,25 @@ constexpr int hex_modal_elems(int nm)
 // 1.6 M points: FP64 NM, NQ = 6, 8 35.5/23.2; 7, 8 37/25; 8, 9 28/39; 8, 10
 // 41/32; 9, 10 42/37; 10, 11 47/34; 10, 12 47/38; 8, 8 40/26; 10, 10 44/39;
 // 6, 7 27/27; 5, 7 26/26; FP32 7, 8 16.8/15.8; 8, 8 17.5/14.8; 8, 10 21/22;
-// 10, 11 23/19; 10, 12 25/20.
-constexpr int hex_deformed_tile(int nm, int nq, bool fp32)
+// 10, 11 23/19; 10, 12 25/20.  The mapped form of the general solver gains as
+// much (apply and assembly, FP64, 7, 8 at 512 / 4,096 elements 18.7/14.0,
+// 52.4/46.3; 10, 11 at 512 / 1,000 34.5/26.2, 43/39.9).  In FP32 at NQ = 11
+// the card holds 1,536 elements at once on the matrix cores and 2,048 on the
+// vector units: the former are faster while they need no more rounds (10, 11,
+// vector / matrix cores at 1,536, 1,552, 2,048, 2,064, 3,072, 4,096, 4,112 and
+// 6,144 elements: 1.07, 0.93, 0.89, 1.22, 1.07, 0.97, 1.14, 0.93).
+constexpr int hex_deformed_tile(int nm, int nq, bool fp32, int nelmt)
 {
-    const bool mfma = nm >= 6 && (fp32 ? nq == 8 || nq >= 11 : nq == 8 || nq >= 10);
+    const auto rounds = [&](int held) { return (nelmt + held - 1) / held; };
+    const bool mfma = nm >= 6 && (fp32 ? nq == 8 || nq == 12 || (nq == 11 && rounds(1536) == rounds(2048))
+                                       : nq == 8 || nq >= 10);
     return mfma ? kMfmaTile + 1 : hex_fill_elems(nq);
 }
-// elements per workgroup of a tile (0: the default) of a hex Helmholtz kind
-inline int hex_tile_elems(int nm, int nq, bool deformed, bool fp32, int tile)
+// elements per workgroup of a tile of a hex Helmholtz kind (0, the default,
+// with affine elements only)
+inline int hex_tile_elems(int nm, int tile)
 {
-    if (tile <= 0 && !deformed) return hex_modal_elems(nm);
-    if (tile <= 0) tile = hex_deformed_tile(nm, nq, fp32);
+    if (tile <= 0) return hex_modal_elems(nm);
     return tile >= kMfmaTile ? tile - kMfmaTile : tile;
 }
 constexpr int tet_packed_tpe(int nq0) { return nq0 * (nq0 - 1); }

@@ -35,3 +35,35 @@ def test_default_tile(nmf, nm, nq, fp32):
     torch.cuda.synchronize()
     for it, y in zip(items, ref):
         assert np.array_equal(it.got()[0], y), it.nelmt
+
+
+def test_single_precision_line_in_elements(nmf):
+    """FP32 at NQ = 11: matrix cores (tile TILE_MFMA + 1) as long as they need
+    no more rounds over the card than the vector tile (2 elements); the two sum
+    in other orders, so the bits tell which one ran."""
+    nm, nq, nqt = 9, 11, 11 ** 3
+    rng = np.random.default_rng(6)
+    batch, alone = nmf.Batch(mode=nmf.Batch.GROUPED), []
+    for nel, tile in ((1536, nmf.TILE_MFMA + 1), (1537, 2), (2048, 2), (2049, nmf.TILE_MFMA + 1)):
+        op = nmf.GetOperatorFactory().CreateInstance("Helmholtz_Hex_Deformed", nm, nq, nel, nmf.FP32)
+        op.SetJac(rng.uniform(0.5, 1.5, nel * nqt))
+        op.SetDF(np.tile(np.eye(3).reshape(-1), nel * nqt) + rng.uniform(-0.2, 0.2, nel * nqt * 9))
+        op.SetLambda(0.7)
+        x = torch.from_numpy(rng.uniform(-1, 1, nel * nm ** 3)).float().cuda()
+        got = {}
+        for t in (0, nmf.TILE_MFMA + 1, 2):
+            op.tile = t
+            got[t] = torch.zeros_like(x)
+            op(x, got[t])
+        op.tile = 0
+        torch.cuda.synchronize()
+        assert not torch.equal(got[nmf.TILE_MFMA + 1], got[2])
+        assert torch.equal(got[0], got[tile]), nel
+        y = torch.zeros_like(x)
+        batch.add(op, x, y)
+        alone.append((got[0], y))
+    assert batch.info()["groups"] == 2
+    batch.run()
+    torch.cuda.synchronize()
+    for want, y in alone:
+        assert torch.equal(want, y)
