@@ -305,8 +305,9 @@ void HexSolver::capture_iterations()
         NMF_HIP(solver::launch_cg_step(stream_, n_, nm_, N_, st, sloc64_.as<double>(), p, q, x, r, w,
                                        invd_.as<double>(), pa_.as<double>()));
         apply_local(false, w, sloc64_.get(), done);
-        NMF_HIP(solver::launch_cg_scalar(stream_, st, pa_.as<double>(), solver::cg_step_blocks(N_),
-                                         edot_.as<double>(), nelmt_));
+        const auto sw = solver::sum_element_dots(stream_, st, nelmt_, edot_.as<double>(), pmu_.as<double>());
+        NMF_HIP(sw.err);
+        NMF_HIP(solver::launch_cg_scalar(stream_, st, pa_.as<double>(), solver::cg_step_blocks(N_), sw.p, sw.n));
     }
     NMF_HIP(hipStreamEndCapture(stream_, &g));
     hipError_t e = hipGraphInstantiate(&graph_[0], g, nullptr, nullptr, 0);
@@ -395,7 +396,9 @@ void HexSolver::begin_solve_enqueue(bool mixed, double tol, int maxit)
         NMF_HIP(solver::launch_cg_init<double>(stream_, N_, b_.as<double>(), invd_.as<double>(), x, r, p, q, w,
                                                pa_.as<double>()));
         apply_local(false, w, sloc64_.get(), nullptr);
-        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, pa_.as<double>(), nb_, edot_.as<double>(), nelmt_));
+        const auto sw = solver::sum_element_dots(stream_, nullptr, nelmt_, edot_.as<double>(), pmu_.as<double>());
+        NMF_HIP(sw.err);
+        NMF_HIP(solver::launch_cg_scalar_init(stream_, st, pa_.as<double>(), nb_, sw.p, sw.n));
         capture_iterations();
         job_.max_rounds = maxit / kItersPerGraph + 3;
     } else {

@@ -664,6 +664,19 @@ __device__ __forceinline__ void reduce_scalars(const double *__restrict__ pa, in
     }
 }
 
+// Sums of the element dots by workgroup, for more elements than the scalar
+// step's one block reads in good time; fixed order.
+__global__ __launch_bounds__(kBlock) void element_dots_kernel(const CGState *__restrict__ st, int nelmt,
+                                                              const double *__restrict__ edot,
+                                                              double *__restrict__ partials)
+{
+    if (st && st->done) return;
+    double v[1] = {0.0};
+    for (size_t e = blockIdx.x * (size_t)kBlock + threadIdx.x; e < (size_t)nelmt; e += (size_t)gridDim.x * kBlock)
+        v[0] += edot[e];
+    block_sum<1>(v, partials + blockIdx.x);
+}
+
 __global__ __launch_bounds__(kScalarBlock) void cg_scalar_init_kernel(CGState *st, const double *__restrict__ pa,
                                                                       int nb, const double *__restrict__ pmu, int nmu)
 {
@@ -1077,6 +1090,14 @@ hipError_t launch_cg_step(hipStream_t stream, int n, int nm, int N, const CGStat
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+ElementDots sum_element_dots(hipStream_t stream, const CGState *st, int nelmt, const double *edot, double *partials)
+{
+    if (nelmt <= kDirectDots) return {edot, nelmt, hipSuccess};
+    const int per = 8 * kBlock, blocks = (nelmt - 1) / per + 1, grid = blocks < kRedBlocks ? blocks : kRedBlocks;
+    NMF_LAUNCH(element_dots_kernel, grid, st, nelmt, edot, partials);
+    return {partials, grid, hipGetLastError()};
 }
 
 hipError_t launch_cg_scalar_init(hipStream_t stream, CGState *st, const double *pa, int nb, const double *pmu,

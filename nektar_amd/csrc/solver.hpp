@@ -55,6 +55,18 @@ hipError_t launch_cg_init(hipStream_t, int N, const double *b, const double *inv
 hipError_t launch_cg_step(hipStream_t, int n, int nm, int N, const CGState *st, const double *sloc, double *p,
                           double *q, double *x, double *r, double *w, const double *inv_diag, double *partials);
 int cg_step_blocks(int N);  // its partials
+// s.w as the scalar steps read it: the element dots themselves, or their sums
+// by workgroup (`partials`, at most kRedBlocks; st: skipped once done, or
+// NULL).  One block reads some 80 GB/s and a launch takes about 2 us; iteration,
+// us, dots read directly / summed first, affine at NM = 2: 28^3 17.9/18.9, 32^3
+// 21.4/22.3, 40^3 25.2/22.2, 64^3 56/34, 128^3 390/172, 200^3 1802/648.
+constexpr int kDirectDots = 1 << 15;
+struct ElementDots {
+    const double *p;
+    int n;
+    hipError_t err;
+};
+ElementDots sum_element_dots(hipStream_t, const CGState *st, int nelmt, const double *edot, double *partials);
 // nb partials of the vector dots, nmu of s.w
 hipError_t launch_cg_scalar_init(hipStream_t, CGState *st, const double *pa, int nb, const double *pmu, int nmu);
 hipError_t launch_cg_scalar(hipStream_t, CGState *st, const double *pa, int nb, const double *pmu, int nmu);

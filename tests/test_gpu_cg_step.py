@@ -25,18 +25,29 @@ def nmf():
     return nektar_amd
 
 
+def check_true_residual(s, n, nm):
+    s.set_forcing_manufactured(1)
+    info = s.solve(tol=1e-10, maxit=8000)
+    assert info.converged, (n, info.as_dict())
+    x = torch.from_numpy(s.solution()).cuda()
+    y = torch.zeros_like(x)
+    s.apply_global(x, y)
+    torch.cuda.synchronize()
+    b, N = s.rhs().reshape((n * (nm - 1) + 1,) * 3), n * (nm - 1) + 1
+    res = (b - y.cpu().numpy().reshape(b.shape))[1:N - 1, 1:N - 1, 1:N - 1]
+    assert np.linalg.norm(res) <= 1.1e-9 * np.linalg.norm(b), (n, np.linalg.norm(res) / np.linalg.norm(b))
+
+
 @pytest.mark.parametrize("nm", range(2, 11))
 @pytest.mark.parametrize("perturb", [0.0, 0.1], ids=["affine", "perturbed"])
 def test_true_residual(nmf, nm, perturb):
     for n in (2, 3, 13 if nm == 6 else 7 if nm < 9 else 4):
-        s = nmf.HelmholtzSolver(n, nm, nm + 1, 1.3, perturb=perturb, seed=3)
-        s.set_forcing_manufactured(1)
-        info = s.solve(tol=1e-10, maxit=8000)
-        assert info.converged, (n, info.as_dict())
-        x = torch.from_numpy(s.solution()).cuda()
-        y = torch.zeros_like(x)
-        s.apply_global(x, y)
-        torch.cuda.synchronize()
-        b, N = s.rhs().reshape((n * (nm - 1) + 1,) * 3), n * (nm - 1) + 1
-        res = (b - y.cpu().numpy().reshape(b.shape))[1:N - 1, 1:N - 1, 1:N - 1]
-        assert np.linalg.norm(res) <= 1.1e-9 * np.linalg.norm(b), (n, np.linalg.norm(res) / np.linalg.norm(b))
+        check_true_residual(nmf.HelmholtzSolver(n, nm, nm + 1, 1.3, perturb=perturb, seed=3), n, nm)
+
+
+@pytest.mark.parametrize("n", [32, 33])
+@pytest.mark.parametrize("perturb", [0.0, 0.1], ids=["affine", "perturbed"])
+def test_true_residual_around_the_direct_sum(nmf, n, perturb):
+    """Up to 32^3 elements the scalar step adds the element dots itself, above
+    it adds their sums by workgroup."""
+    check_true_residual(nmf.HelmholtzSolver(n, 2, 3, 1.3, perturb=perturb, seed=3), n, 2)
