@@ -58,8 +58,8 @@ int cg_step_blocks(int N);  // its partials
 // s.w as the scalar steps read it: the element dots themselves, or their sums
 // by workgroup (`partials`, at most kRedBlocks; st: skipped once done, or
 // NULL).  One block reads some 80 GB/s and a launch takes about 2 us; iteration,
-// us, dots read directly / summed first, affine at NM = 2: 28^3 17.9/18.9, 32^3
-// 21.4/22.3, 40^3 25.2/22.2, 64^3 56/34, 128^3 390/172, 200^3 1802/648.
+// us, dots read directly / summed first, affine at NM = 2: 32^3
+// 21.1/21.5, 40^3 25.2/20.5, 64^3 56/32, 128^3 390/172, 200^3 1802/649.
 constexpr int kDirectDots = 1 << 15;
 struct ElementDots {
     const double *p;
