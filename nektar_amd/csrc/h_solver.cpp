@@ -244,7 +244,7 @@ void HexSolver::autotune(int *tile64, int *tile32, std::vector<double> *times64,
     for (int prec = 0; prec < 2; ++prec) {
         const bool fp32 = prec == 1;
         int buf[8];
-        const int nc = hex_tile_candidates(nm_, nq_, fp32, buf, 8);
+        const int nc = hex_tile_candidates(nm_, nq_, fp32, deformed_, buf, 8);
         std::vector<int> cand(buf, buf + nc);
         // a scratch global vector of non-zero normal values (every byte
         // 0x3F) serves as input, so the timed arithmetic draws real power

@@ -56,7 +56,7 @@ struct SolverArgs {
 
 // Tile shapes (elements per workgroup) available for the hex Helmholtz
 // kernels of a given order, in the order the autotuner tries them.
-int hex_tile_candidates(int nm, int nq, bool fp32, int *out, int max);
+int hex_tile_candidates(int nm, int nq, bool fp32, bool deformed, int *out, int max);
 
 // Grouped Helmholtz: several operators of one kind (shape, modes, points,
 // precision, geometry type) in one launch.  Items are ordered with

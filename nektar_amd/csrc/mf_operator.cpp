@@ -565,7 +565,7 @@ std::vector<int> MFOperator::tile_candidates() const
     std::vector<int> c;
     if (generic || op == OpType::PhysInterp) return c;
     int buf[8], n = 0;
-    if (shape == Shape::Hex && op == OpType::Helmholtz) n = hex_tile_candidates(nm, nq[0], fp32, buf, 8);
+    if (shape == Shape::Hex && op == OpType::Helmholtz) n = hex_tile_candidates(nm, nq[0], fp32, deformed, buf, 8);
     if (shape == Shape::Tet) n = tet_tile_candidates(nq[0], buf, 8);
     c.assign(buf, buf + n);
     return c;

@@ -56,3 +56,28 @@ def test_against_oracle_around_a_workgroup(nmf, nm, nq, fp32):
         ref = O.helmholtz(O.HEX, nm, nq, nel, False, jac, df, 0.7, x, diff6)
         err = np.max(np.abs(got[:nel * nm ** 3] - ref)) / np.max(np.abs(ref))
         assert err <= (2e-5 if fp32 else 1e-12), (nel, err)
+
+
+@pytest.mark.parametrize("nm,nq", [(nm, nm + d) for nm in range(2, 11) for d in (1, 2)])
+@pytest.mark.parametrize("fp32", [False, True], ids=["fp64", "fp32"])
+def test_default_tile_is_a_candidate(nmf, nm, nq, fp32):
+    """The autotuner can choose the default's elements per workgroup, alone and
+    in a batch, and gets the default's results."""
+    per = 64 // nm ** 2 if nm <= 4 else 5 if nm <= 6 else 2 if nm == 9 else 1
+    nel, dt = 2 * per + 1, torch.float32 if fp32 else torch.float64
+    jac, df = sheared(nel, nm)
+    op = nmf.GetOperatorFactory().CreateInstance("Helmholtz_Hex_Regular", nm, nq, nel, nmf.FP32 if fp32 else nmf.FP64)
+    op.SetJac(jac)
+    op.SetDF(df)
+    op.SetLambda(0.7)
+    assert op.tile == 0 and per in op.tile_candidates()
+    x = torch.from_numpy(O.splitmix_uniform(nel, nel * nm ** 3)).to(dt).cuda()
+    default, pinned, grouped = torch.zeros_like(x), torch.zeros_like(x), torch.zeros_like(x)
+    op(x, default)
+    op.tile = per
+    op(x, pinned)
+    batch = nmf.Batch(mode=nmf.Batch.GROUPED)
+    batch.add(op, x, grouped)
+    batch.run()
+    torch.cuda.synchronize()
+    assert torch.equal(default, pinned) and torch.equal(default, grouped)
