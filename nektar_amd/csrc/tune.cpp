@@ -1,11 +1,11 @@
 #include "tune.hpp"
 
-#include <limits>
 #include <map>
 #include <mutex>
 #include <tuple>
 
 #include "common.hpp"
+#include "tune_pick.hpp"
 
 namespace nektar_amd {
 
@@ -51,29 +51,20 @@ int time_tiles(hipStream_t s, const std::vector<int> &candidates, const std::fun
     hipEvent_t e0, e1;
     NMF_HIP(hipEventCreate(&e0));
     NMF_HIP(hipEventCreate(&e1));
-    int best = 0;
-    double best_t = std::numeric_limits<double>::infinity();
-    if (times_us) times_us->assign(candidates.size(), std::numeric_limits<double>::infinity());
-    for (size_t c = 0; c < candidates.size(); ++c) {
-        const int t = candidates[c];
+    const auto sample = [&](int t) {
         if (launch(t) != hipSuccess) {
             (void)hipGetLastError();
-            continue;
+            return -1.0;
         }
-        for (int w = 0; w < 2; ++w) NMF_HIP(launch(t));
         NMF_HIP(hipEventRecord(e0, s));
         for (int r = 0; r < reps; ++r) NMF_HIP(launch(t));
         NMF_HIP(hipEventRecord(e1, s));
         NMF_HIP(hipEventSynchronize(e1));
         float ms = 0.f;
         NMF_HIP(hipEventElapsedTime(&ms, e0, e1));
-        const double us = 1e3 * ms / reps;
-        if (times_us) (*times_us)[c] = us;
-        if (us < best_t) {
-            best_t = us;
-            best = t;
-        }
-    }
+        return 1e3 * ms / reps;
+    };
+    const int best = pick_tile(candidates, sample, times_us);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     NMF_REQUIRE(best > 0, NMF_ERR_DEVICE, "every tile candidate failed to launch");

@@ -23,9 +23,10 @@ void record_tile(const TuneKey &k, int tile);
 void clear_tuned_tiles();
 
 // Times launch(tile) for every candidate (warm-up, then `reps` launches
-// between two events on `s`) and returns the fastest tile; per-candidate
-// mean times in microseconds go to times_us when given.  A candidate whose
-// launch fails is skipped.
+// between two events on `s`, again for those near the fastest: tune_pick.hpp)
+// and returns the fastest tile; the shortest mean time of each candidate in
+// microseconds goes to times_us when given.  A candidate whose launch fails is
+// skipped.
 int time_tiles(hipStream_t s, const std::vector<int> &candidates, const std::function<hipError_t(int)> &launch,
                int reps, std::vector<double> *times_us = nullptr);
 
