@@ -219,8 +219,9 @@ int nmf_operator_apply_physderiv_host(nmf_operator op, const double *in,
  * kernel for two (work-items per element: nq0*(nq0-1), elements sharing
  * waves, or that rounded up to a multiple of 64, one element per wave at
  * nq0 <= 8), and the fastest is measured per (key, nummodes, numpoints,
- * precision) on the caller's data.  The choice is remembered for the rest of the process:
- * operators and solvers created later for the same kind start from it.
+ * precision) on the caller's data.  The choice is remembered for the rest of
+ * the process: operators and solvers created later for the same kind, with at
+ * most four times the elements, start from it.
  * tile 0 = the library default.  Results do not depend on the tile,
  * except that hex Helmholtz tiles NMF_TILE_MFMA + E (E = 1, 2, 4 elements
  * per workgroup, NUMMODES >= 5) run the per-direction products on the

@@ -142,8 +142,8 @@ HexSolver::HexSolver(const HexBoxMesh &mesh, int nummodes, int numpoints, double
     NMF_HIP(hipEventCreate(&ev_t1_));
     build_geometry();
     build_diagonal();
-    tile64_ = tuned_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, 0, deformed_ ? 1 : 0, 1});
-    tile32_ = tuned_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, 1, deformed_ ? 1 : 0, 1});
+    tile64_ = tuned_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, 0, deformed_ ? 1 : 0, 1}, nelmt_);
+    tile32_ = tuned_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, 1, deformed_ ? 1 : 0, 1}, nelmt_);
     NMF_HIP(hipStreamSynchronize(stream_));
 }
 
@@ -262,7 +262,8 @@ void HexSolver::autotune(int *tile64, int *tile32, std::vector<double> *times64,
             },
             10, fp32 ? times32 : times64);
         (fp32 ? tile32_ : tile64_) = best;
-        record_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, prec, deformed_ ? 1 : 0, 1}, best);
+        record_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, prec, deformed_ ? 1 : 0, 1},
+                    nelmt_, best);
     }
     for (auto &g : graph_)
         if (g) {

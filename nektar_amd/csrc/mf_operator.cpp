@@ -154,7 +154,7 @@ void MFOperator::init(const std::string &key, const int nummodes[3], const int n
     }
     if (op == OpType::BwdTrans || op == OpType::PhysInterp) deformed = false;  // no geometry
     if (op == OpType::PhysInterp) set_scaling_factor(1.5);  // the reference's default (Operator.hpp:136-141)
-    if (!generic) tile = tuned_tile(tune_key());
+    if (!generic) tile = tuned_tile(tune_key(), nelmt);
 }
 
 void MFOperator::prepare()
@@ -611,7 +611,7 @@ int MFOperator::autotune(hipStream_t s, std::vector<double> *times_us)
         10, times_us);
     tile = best;
     ++version;
-    record_tile(tune_key(), best);
+    record_tile(tune_key(), nelmt, best);
     return best;
 }
 

@@ -17,24 +17,30 @@ bool TuneKey::operator<(const TuneKey &o) const
 
 namespace {
 std::mutex g_tune_mutex;
-std::map<TuneKey, int> &tune_table()
+// by the element count of the measurement
+std::map<TuneKey, std::map<int, int>> &tune_table()
 {
-    static std::map<TuneKey, int> t;
+    static std::map<TuneKey, std::map<int, int>> t;
     return t;
 }
 }  // namespace
 
-int tuned_tile(const TuneKey &k)
+int tuned_tile(const TuneKey &k, int nelmt)
 {
     std::lock_guard<std::mutex> l(g_tune_mutex);
     auto it = tune_table().find(k);
-    return it == tune_table().end() ? 0 : it->second;
+    if (it == tune_table().end()) return 0;
+    const auto &by_count = it->second;
+    const auto larger = by_count.lower_bound(nelmt);
+    if (larger != by_count.end()) return larger->second;
+    const auto &largest = *by_count.rbegin();
+    return nelmt / kTunedReach <= largest.first ? largest.second : 0;
 }
 
-void record_tile(const TuneKey &k, int tile)
+void record_tile(const TuneKey &k, int nelmt, int tile)
 {
     std::lock_guard<std::mutex> l(g_tune_mutex);
-    tune_table()[k] = tile;
+    tune_table()[k][nelmt] = tile;
 }
 
 void clear_tuned_tiles()

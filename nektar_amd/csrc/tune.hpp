@@ -2,7 +2,8 @@
 // Helmholtz kernels is chosen per (shape, operator, order, points,
 // precision, geometry, input form) by timing every instantiated tile on
 // the caller's own data, and remembered for the rest of the process so
-// later operators of the same kind start from the measured choice.
+// later operators of the same kind start from the measured choice, if they
+// are not much larger than what was measured.
 #pragma once
 
 #include <functional>
@@ -17,9 +18,15 @@ struct TuneKey {
     bool operator<(const TuneKey &o) const;
 };
 
-// 0 when nothing has been measured for the key.
-int tuned_tile(const TuneKey &k);
-void record_tile(const TuneKey &k, int tile);
+// The choice measured on nelmt elements or the next larger count, else on the
+// largest one if nelmt is at most kTunedReach times that; 0 when there is none.
+// What wins on a collection that leaves CUs idle can lose on one that does not:
+// chosen on 64 elements and run on some 10 M coefficients, affine hexes at
+// NM = 3 and 6 take 1.2 times the default's time, curved ones, FP64 at NM = 8
+// 1.4 times and FP32 at NM = 5 1.6 times.
+constexpr int kTunedReach = 4;
+int tuned_tile(const TuneKey &k, int nelmt);
+void record_tile(const TuneKey &k, int nelmt, int tile);
 void clear_tuned_tiles();
 
 // Times launch(tile) for every candidate (warm-up, then `reps` launches

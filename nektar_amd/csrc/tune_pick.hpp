@@ -12,7 +12,7 @@ namespace nektar_amd {
 // one timing of t in us, negative if t cannot run.  A single timing of a short
 // kernel is off by several per cent, and the first ones more (the clocks are
 // still low), so every candidate within 1.25 of the shortest is timed again,
-// kRounds times in all and in turn, and the shortest counts; a tie goes to the
+// kTuneRounds times in all and in turn, and the shortest counts; a tie goes to the
 // earlier candidate.  15 kinds of hexes, 500 to 90,000 elements, tuned six
 // times each: with one timing a choice up to 5 % slower than the default, with
 // these up to 0.6 %.

@@ -104,6 +104,26 @@ def test_autotune_records_choice(nmf):
     assert op4.tile == 0
 
 
+def test_recorded_choice_reaches_four_times_the_elements(nmf):
+    nmf.clear_tuning()
+
+    def op(n):
+        return _op(nmf, 4, 5, n, False, False)[0]
+
+    small = op(4)
+    best, _ = small.autotune()
+    assert best > 0 and small.tile == best
+    assert op(3).tile == best and op(6).tile == best  # 27 and 216 of 64 elements
+    assert op(7).tile == 0                            # 343
+    large = op(12)
+    large.tile = 0
+    best_large, _ = large.autotune()
+    assert op(7).tile == best_large and op(12).tile == best_large
+    assert op(4).tile == best                         # the nearest count at or above
+    nmf.clear_tuning()
+    assert op(4).tile == 0
+
+
 def test_solver_autotune_keeps_iterates(nmf):
     nmf.clear_tuning()
     s = nmf.HelmholtzSolver(4, 5, 6, 1.0, perturb=0.1, seed=5)
