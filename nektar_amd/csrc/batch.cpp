@@ -129,10 +129,13 @@ void Batch::build()
             singles_.push_back(i);
             continue;
         }
+        // the tile that runs: affine tets have one kernel for every tile, and
         // the default of curved hexes depends on the member's size
-        const int tile = o.tile == 0 && o.shape == Shape::Hex && o.deformed
-                             ? hex_deformed_tile(o.nm, o.nq[0], o.fp32, o.nelmt)
-                             : o.tile;
+        int tile = o.tile;
+        if (o.shape == Shape::Tet && !o.deformed)
+            tile = 0;
+        else if (tile == 0 && o.shape == Shape::Hex && o.deformed)
+            tile = hex_deformed_tile(o.nm, o.nq[0], o.fp32, o.nelmt);
         const auto key = std::make_tuple((int)o.shape, o.nm, o.nq[0], tile, (int)o.fp32, (int)o.deformed);
         auto it = index.find(key);
         if (it == index.end()) {

@@ -87,3 +87,23 @@ def test_both_variants_alone_and_grouped(nmf, nm, fp32):
     torch.cuda.synchronize()
     for y, grouped in outs:
         assert torch.equal(y, grouped)
+
+
+def test_one_group_whatever_the_tile(nmf):
+    """One kernel serves every tile of affine tets, so members with different
+    tiles share a launch."""
+    batch = nmf.Batch(mode=nmf.Batch.GROUPED)
+    outs = []
+    for k, nel in enumerate((5, 70, 33)):
+        op, _, _ = operator(nmf, 4, 5, nel, False, None)
+        op.tile = ([0] + op.tile_candidates())[k]
+        x = torch.from_numpy(O.splitmix_uniform(nel, nel * 20)).cuda()
+        y, grouped = torch.zeros_like(x), torch.zeros_like(x)
+        op(x, y)
+        batch.add(op, x, grouped)
+        outs.append((y, grouped))
+    assert batch.info()["groups"] == 1
+    batch.run()
+    torch.cuda.synchronize()
+    for y, grouped in outs:
+        assert torch.equal(y, grouped)

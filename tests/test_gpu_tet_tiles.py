@@ -3,8 +3,10 @@ element, elements sharing waves) and wave-aligned (rounded up to a
 multiple of 64, so that at Q <= 8 every element is one wave that
 synchronises only itself).
 
-Both tiles run the same arithmetic in the same order, so every operator's
-output must be bit-identical between them; the FP64 output is checked
+Both tiles run the same arithmetic in the same order (the affine Helmholtz
+operator one and the same kernel, whose two variants go by the element count:
+test_gpu_tet_modal.py), so every operator's output must be bit-identical
+between them; the FP64 output is checked
 against the oracle (relative max error <= 1e-12) and FP32 at 2e-5 (2e-4
 above 7 modes).  The element counts leave a ragged last workgroup for both
 tiles."""
