@@ -337,6 +337,9 @@ int nmf_solver_apply_global(nmf_solver s, const double *x_dev, double *y_dev);
 /* Autotune the solver's gather-apply kernel (FP64 and FP32 iterations);
  * iteration graphs are re-captured on the next solve. */
 int nmf_solver_autotune(nmf_solver s, int *tile64, int *tile32);
+/* Pin the tiles instead (candidates of the Helmholtz operator of the same
+ * kind and precision; 0 = the library default). */
+int nmf_solver_set_tiles(nmf_solver s, int tile64, int tile32);
 /* Forget every tile the autotuner recorded in this process. */
 int nmf_clear_tuning(void);
 /* ---------------------------------------------------------------------

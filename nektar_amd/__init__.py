@@ -103,6 +103,7 @@ _SIGNATURES = {
     "nmf_operator_get_tile": (ctypes.c_int, [_P, _I]),
     "nmf_operator_autotune": (ctypes.c_int, [_P, _P, _I, _D, ctypes.c_int]),
     "nmf_solver_autotune": (ctypes.c_int, [_P, _I, _I]),
+    "nmf_solver_set_tiles": (ctypes.c_int, [_P, ctypes.c_int, ctypes.c_int]),
     "nmf_server_create": (ctypes.c_int, [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.POINTER(_P)]),
     "nmf_server_destroy": (ctypes.c_int, [_P]),
     "nmf_server_run": (ctypes.c_int, [_P, _P, ctypes.c_int, ctypes.c_int, _P, _P]),
@@ -611,6 +612,10 @@ class HelmholtzSolver:
         t64, t32 = ctypes.c_int(), ctypes.c_int()
         check(lib().nmf_solver_autotune(self._h, ctypes.byref(t64), ctypes.byref(t32)))
         return t64.value, t32.value
+
+    def set_tiles(self, tile64: int = 0, tile32: int = 0) -> None:
+        """Pin the gather-apply tiles instead (0: the default)."""
+        check(lib().nmf_solver_set_tiles(self._h, tile64, tile32))
 
     def l2_error_manufactured(self, k: int = 1) -> float:
         v = ctypes.c_double()

@@ -634,6 +634,14 @@ int nmf_solver_autotune(nmf_solver s, int *tile64, int *tile32)
     });
 }
 
+int nmf_solver_set_tiles(nmf_solver s, int tile64, int tile32)
+{
+    return guard([&] {
+        NMF_REQUIRE(s && s->impl, NMF_ERR_INVALID, "null solver handle");
+        s->impl->set_tiles(tile64, tile32);
+    });
+}
+
 int nmf_clear_tuning(void)
 {
     return guard([&] { clear_tuned_tiles(); });

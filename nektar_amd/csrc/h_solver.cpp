@@ -237,15 +237,43 @@ void HexSolver::apply_local(bool fp32, const void *xg, void *sloc, const int *do
     NMF_HIP(launch_hex_solver(nm_, nq_, a));
 }
 
+std::vector<int> HexSolver::tile_candidates(bool fp32) const
+{
+    int buf[8];
+    const int n = hex_tile_candidates(nm_, nq_, fp32, deformed_, buf, 8);
+    return std::vector<int>(buf, buf + n);
+}
+
+void HexSolver::drop_graphs()
+{
+    for (auto &g : graph_)
+        if (g) {
+            NMF_HIP(hipGraphExecDestroy(g));
+            g = nullptr;
+        }
+}
+
+void HexSolver::set_tiles(int tile64, int tile32)
+{
+    NMF_REQUIRE(!job_.running, NMF_ERR_STATE, "set_tiles during a solve");
+    for (const bool fp32 : {false, true}) {
+        const int t = fp32 ? tile32 : tile64;
+        const auto cand = tile_candidates(fp32);
+        NMF_REQUIRE(t == 0 || std::find(cand.begin(), cand.end(), t) != cand.end(), NMF_ERR_INVALID,
+                    "tile " + std::to_string(t) + " is not instantiated for this solver");
+    }
+    tile64_ = tile64;
+    tile32_ = tile32;
+    drop_graphs();
+}
+
 void HexSolver::autotune(int *tile64, int *tile32, std::vector<double> *times64, std::vector<double> *times32)
 {
     NMF_REQUIRE(!job_.running, NMF_ERR_STATE, "autotune during a solve");
     ensure_fp32();
     for (int prec = 0; prec < 2; ++prec) {
         const bool fp32 = prec == 1;
-        int buf[8];
-        const int nc = hex_tile_candidates(nm_, nq_, fp32, deformed_, buf, 8);
-        std::vector<int> cand(buf, buf + nc);
+        const std::vector<int> cand = tile_candidates(fp32);
         // a scratch global vector of non-zero normal values (every byte
         // 0x3F) serves as input, so the timed arithmetic draws real power
         void *xg = fp32 ? cg32_[2].get() : tmp64_.get();
@@ -265,11 +293,7 @@ void HexSolver::autotune(int *tile64, int *tile32, std::vector<double> *times64,
         record_tile(TuneKey{(int)Shape::Hex, (int)OpType::Helmholtz, nm_, nq_, prec, deformed_ ? 1 : 0, 1},
                     nelmt_, best);
     }
-    for (auto &g : graph_)
-        if (g) {
-            NMF_HIP(hipGraphExecDestroy(g));
-            g = nullptr;
-        }
+    drop_graphs();
     if (tile64) *tile64 = tile64_;
     if (tile32) *tile32 = tile32_;
 }
@@ -536,11 +560,7 @@ void HexSolver::set_lambda(double lambda)
     lambda_ = lambda;
     build_diagonal();
     // the captured iterations carry lambda as a kernel argument
-    for (auto &g : graph_)
-        if (g) {
-            NMF_HIP(hipGraphExecDestroy(g));
-            g = nullptr;
-        }
+    drop_graphs();
 }
 
 double HexSolver::solution_norm()

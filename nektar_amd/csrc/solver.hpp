@@ -194,6 +194,8 @@ public:
     // rebuilt on the next solve.
     void autotune(int *tile64, int *tile32, std::vector<double> *times64 = nullptr,
                   std::vector<double> *times32 = nullptr);
+    // Pin them instead (0: the default)
+    void set_tiles(int tile64, int tile32);
     int tile(bool fp32) const { return fp32 ? tile32_ : tile64_; }
 
     size_t nglobal() const { return NG_; }
@@ -218,6 +220,8 @@ private:
     void apply_local(bool fp32, const void *xg, void *sloc, const int *done);
     void apply_global_fp64(const double *x, double *y);  // no state check (used inside solves)
     void capture_iterations();
+    std::vector<int> tile_candidates(bool fp32) const;
+    void drop_graphs();
     void assemble_rhs(const double *f_dev);
     void enqueue_state_read();
     void enqueue_reliable_update();

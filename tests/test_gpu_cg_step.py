@@ -25,9 +25,9 @@ def nmf():
     return nektar_amd
 
 
-def check_true_residual(s, n, nm):
+def check_true_residual(s, n, nm, mixed=False):
     s.set_forcing_manufactured(1)
-    info = s.solve(tol=1e-10, maxit=8000)
+    info = s.solve(mixed, tol=1e-10, maxit=8000)
     assert info.converged, (n, info.as_dict())
     x = torch.from_numpy(s.solution()).cuda()
     y = torch.zeros_like(x)
@@ -51,3 +51,28 @@ def test_true_residual_around_the_direct_sum(nmf, n, perturb):
     """Up to 32^3 elements the scalar step adds the element dots itself, above
     it adds their sums by workgroup."""
     check_true_residual(nmf.HelmholtzSolver(n, 2, 3, 1.3, perturb=perturb, seed=3), n, 2)
+
+
+@pytest.mark.parametrize("nm,d", [(2, 1), (2, 2), (3, 1), (4, 2), (5, 1), (5, 2), (6, 2), (7, 1), (8, 2), (9, 1), (10, 1),
+                                  (10, 2)])
+@pytest.mark.parametrize("perturb", [0.0, 0.1], ids=["affine", "perturbed"])
+def test_true_residual_of_every_tile(nmf, nm, d, perturb):
+    """Every producer of the element dots: the gather kernels at each tile, and
+    the separate dot after a matrix-core tile.  The vector tiles do the same
+    sums, so their iterates agree bit for bit, and so do the matrix-core ones."""
+    key = "Helmholtz" + nmf.GetOpstring("Hex", perturb != 0.0)
+    cand = [nmf.GetOperatorFactory().CreateInstance(key, nm, nm + d, 1, p).tile_candidates()
+            for p in (nmf.FP64, nmf.FP32)]
+    for n in (1, 3) if nm > 2 else (2, 5):
+        s = nmf.HelmholtzSolver(n, nm, nm + d, 1.3, perturb=perturb, seed=3)
+        solutions = {}
+        for tile in [0] + cand[0]:
+            s.set_tiles(tile, 0)
+            check_true_residual(s, n, nm)
+            same = solutions.setdefault(tile >= nmf.TILE_MFMA, s.solution())
+            assert np.array_equal(same, s.solution()), tile
+        for tile in cand[1]:
+            s.set_tiles(0, tile)
+            check_true_residual(s, n, nm, mixed=True)
+        with pytest.raises(nmf.NektarError):
+            s.set_tiles(3 if nm not in (9, 10) else 5, 0)
