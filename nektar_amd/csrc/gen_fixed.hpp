@@ -5,9 +5,9 @@
 // The runtime-size kernels spend their time around the products: trip counts
 // and index divisions at run time, every table value a global load of its own,
 // all operators in one kernel.  Here the sizes and the operator are constants
-// (set in the kernel's copy of the arguments, from where they propagate), the
-// tables and index tables are staged in LDS, and a workgroup walks several
-// elements on one staging.  4,096 prisms at NM = 5, NQ = 6: FP64 45.5 -> 19.9 us,
+// (set in the kernel's copy of the arguments, from where they propagate), and
+// every workgroup stages the tables and index tables in LDS (for one element up
+// to kFixedGroups elements, for several above).  4,096 prisms at NM = 5, NQ = 6: FP64 45.5 -> 19.9 us,
 // FP32 38.0 -> 14.8; bound by LDS, which serves every value of a product (a
 // register budget for 6 or 8 waves per SIMD instead of 5 changes nothing, and
 // derivatives line by line, one direction per wave with its matrix in scalar
@@ -21,7 +21,8 @@
 namespace nektar_amd {
 namespace gen {
 
-// workgroups of the walking grid: every CU has as many as its LDS and waves hold
+// workgroups of the walking grid: at least as many as the LDS and waves of the
+// 256 CUs hold
 constexpr int kFixedGroups = 256 * 16;
 
 template <int SH, int NM, int NQ>

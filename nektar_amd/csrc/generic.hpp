@@ -68,7 +68,8 @@ hipError_t launch_generic(const GenArgs &a);
 // the three directions and the default points (Q, Q, Q - 1) with Q = NM + 1 or
 // NM + 2, NM = 3 .. 7.  Prisms, 4,096 elements, FP64 us on the runtime-size
 // kernels and here: NM = 3 26.8/7.2, 4 34.8/12.6, 5 45.5/19.9, 6 70.6/33.3,
-// 7 106/57; 50 elements at NM = 3 9.0/4.3, 7 18.0/9.0.
+// 7 106/57; 50 elements at NM = 3 9.0/4.3, 7 18.0/9.0.  NM = 2 and NM >= 8 are
+// not instantiated: neither was measured.
 constexpr int kFixedMinModes = 3, kFixedMaxModes = 7;
 inline bool fixed_sizes(const GenArgs &a)
 {

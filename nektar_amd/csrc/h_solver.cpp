@@ -356,7 +356,7 @@ void HexSolver::ensure_fp32()
 
 void HexSolver::capture_pcg32()
 {
-    if (graph_[2]) return;
+    if (graph_[1]) return;
     std::lock_guard<std::mutex> lock(graph_capture_mutex());
     CGState *st = state_.as<CGState>();
     const int *done = &st->done;
@@ -374,7 +374,7 @@ void HexSolver::capture_pcg32()
         NMF_HIP(solver::launch_pcg_update_p<float>(stream_, N_, st, r, p, invd32_.as<float>()));
     }
     NMF_HIP(hipStreamEndCapture(stream_, &g));
-    hipError_t e = hipGraphInstantiate(&graph_[2], g, nullptr, nullptr, 0);
+    hipError_t e = hipGraphInstantiate(&graph_[1], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     NMF_REQUIRE(e == hipSuccess, NMF_ERR_DEVICE, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
 }
@@ -527,7 +527,7 @@ bool HexSolver::advance(bool wait)
     if (job_.mixed && st.pause)
         enqueue_reliable_update();
     else
-        NMF_HIP(hipGraphLaunch(graph_[job_.mixed ? 2 : 0], stream_));
+        NMF_HIP(hipGraphLaunch(graph_[job_.mixed ? 1 : 0], stream_));
     ++job_.rounds;
     enqueue_state_read();
     return false;

@@ -314,11 +314,11 @@ __device__ __forceinline__ void deriv2_column(const Tab<T, NM, NQ> &tab, const T
 
 // ===================================================================
 // BwdTrans (BwdTransKernels.hpp:160-227)
-template <typename T, int NM, int NQ, int EPB>
-__global__ __launch_bounds__(EPB * NQ * NQ) void bwdtrans_kernel(
+template <typename T, int NM, int NQ>
+__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void bwdtrans_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ in, T *__restrict__ out)
 {
-    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
+    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
@@ -336,12 +336,12 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void bwdtrans_kernel(
 }
 
 // IProductWRTBase (IProductKernels.hpp:270-350, SCALE=APPEND=false)
-template <typename T, int NM, int NQ, bool DEF, int EPB>
-__global__ __launch_bounds__(EPB * NQ * NQ) void iproduct_kernel(
+template <typename T, int NM, int NQ, bool DEF>
+__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void iproduct_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ jac, const T *__restrict__ in,
     T *__restrict__ out)
 {
-    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
+    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ;
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
@@ -620,12 +620,12 @@ __device__ __forceinline__ void helmholtz_element(const Tab<T, NM, NQ> &tab, con
 // t_d) with t_d = sum_j df[j*3+d] in_j.  Packed geometry: regular
 // g[e*9 + j*3+d] = J df[j*3+d] (weights applied here); deformed
 // g[(e*9 + j*3+d)*Q^3 + q] = W_q J_q df_q[j*3+d].
-template <typename T, int NM, int NQ, bool DEF, int EPB>
-__global__ __launch_bounds__(EPB * NQ * NQ) void iproduct_deriv_kernel(
+template <typename T, int NM, int NQ, bool DEF>
+__global__ __launch_bounds__(elements_per_block<NQ>() * NQ * NQ) void iproduct_deriv_kernel(
     int nelmt, const T *__restrict__ tabp, const T *__restrict__ geo, const T *__restrict__ in0,
     const T *__restrict__ in1, const T *__restrict__ in2, T *__restrict__ out)
 {
-    constexpr int TPE = NQ * NQ, NQ3 = NQ * NQ * NQ, P = pitch<NQ>();
+    constexpr int EPB = elements_per_block<NQ>(), TPE = NQ * NQ, NQ3 = NQ * NQ * NQ, P = pitch<NQ>();
     __shared__ T lds[EPB][2][slab<NQ>()];
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;

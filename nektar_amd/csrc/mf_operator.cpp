@@ -131,7 +131,8 @@ void MFOperator::init(const std::string &key, const int nummodes[3], const int n
     int dq[3];
     default_points(shape, nq[0], dq);
     const bool iso = nmd[1] == nm && nmd[2] == nm && nq[1] == dq[1] && nq[2] == dq[2];
-    // (prisms and pyramids always run the runtime-size kernels)
+    // (prisms and pyramids go through launch_generic, which has compile-time
+    // sizes of its own: fixed_sizes())
     const bool compiled = iso && (shape == Shape::Hex   ? hex_op_supported(nm, nq[0])
                                   : shape == Shape::Tet ? tet_supported(nm, nq[0])
                                                         : false);

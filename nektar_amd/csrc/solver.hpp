@@ -257,7 +257,7 @@ private:
     solver::CGState *host_state_ = nullptr;
     double *host_scalar_ = nullptr;
 
-    hipGraphExec_t graph_[3] = {nullptr, nullptr, nullptr};
+    hipGraphExec_t graph_[2] = {nullptr, nullptr};  // iterations of the FP64 and of the mixed solve
     void capture_pcg32();
     void ensure_fp32();
     static constexpr int kItersPerGraph = 8;

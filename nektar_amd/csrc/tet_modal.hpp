@@ -148,6 +148,21 @@ struct Regs {
     typename hexmf::Mma<T>::v4 ye[L::TE], yo[L::TO];
 };
 
+// Entry s of a parity's vector
+template <bool ODD, int s, typename T, int NM>
+__device__ __forceinline__ T entry(const Regs<T, NM> &R)
+{
+    if constexpr (ODD) return R.xo[s];
+    else return R.xe[s];
+}
+// Its output tile t
+template <bool ODD, int t, typename T, int NM>
+__device__ __forceinline__ typename hexmf::Mma<T>::v4 &tile(Regs<T, NM> &R)
+{
+    if constexpr (ODD) return R.yo[t];
+    else return R.ye[t];
+}
+
 // Coefficient index of entry i of a parity's vector (PARTNER: of the other
 // one of its pair), -1 where there is none
 template <int NM>
@@ -201,12 +216,12 @@ __device__ __forceinline__ void grad_item(Regs<T, NM> &R, S &st, const T (&m)[6]
         constexpr int s = decltype(sc)::value;
         if constexpr (s < S0) {
             constexpr int pos = B.fwd[m0][t][s];
-            if constexpr (pos >= 0) g[0] = M::op(st.template get<pos>(), ODD ? R.xe[s] : R.xo[s], g[0]);
+            if constexpr (pos >= 0) g[0] = M::op(st.template get<pos>(), entry<!ODD, s>(R), g[0]);
         }
         if constexpr (s < S1) {
             constexpr int p1 = B.fwd[m0 + 1][t][s], p2 = B.fwd[m0 + 2][t][s];
-            if constexpr (p1 >= 0) g[1] = M::op(st.template get<p1>(), ODD ? R.xo[s] : R.xe[s], g[1]);
-            if constexpr (p2 >= 0) g[2] = M::op(st.template get<p2>(), ODD ? R.xo[s] : R.xe[s], g[2]);
+            if constexpr (p1 >= 0) g[1] = M::op(st.template get<p1>(), entry<ODD, s>(R), g[1]);
+            if constexpr (p2 >= 0) g[2] = M::op(st.template get<p2>(), entry<ODD, s>(R), g[2]);
         }
     });
 #pragma unroll
@@ -225,12 +240,12 @@ __device__ __forceinline__ void grad_item(Regs<T, NM> &R, S &st, const T (&m)[6]
                 if constexpr (y < T0) {
                     constexpr int pos = B.bwd[m0][y][4 * t + v];
                     if constexpr (pos >= 0) {
-                        auto &acc = ODD ? R.ye[y < L::TE ? y : 0] : R.yo[y < L::TO ? y : 0];
+                        auto &acc = tile<!ODD, y>(R);
                         acc = M::op(st.template get<pos>(), g[0][v], acc);
                     }
                 }
                 if constexpr (y < T1) {
-                    auto &acc = ODD ? R.yo[y < L::TO ? y : 0] : R.ye[y < L::TE ? y : 0];
+                    auto &acc = tile<ODD, y>(R);
                     constexpr int p1 = B.bwd[m0 + 1][y][4 * t + v], p2 = B.bwd[m0 + 2][y][4 * t + v];
                     if constexpr (p1 >= 0) acc = M::op(st.template get<p1>(), g[1][v], acc);
                     if constexpr (p2 >= 0) acc = M::op(st.template get<p2>(), g[2][v], acc);
@@ -248,11 +263,11 @@ __device__ __forceinline__ void mass_item(Regs<T, NM> &R, S &st, T lj)
     constexpr auto &B = L::plan.b;
     for_range<0, (ODD ? L::SO : L::SE)>([&](auto sc) {
         constexpr int s = decltype(sc)::value;
-        const T x = lj * (ODD ? R.xo[ODD ? s : 0] : R.xe[ODD ? 0 : s]);
+        const T x = lj * entry<ODD, s>(R);
         for_range<0, (ODD ? L::TO : L::TE)>([&](auto yc) {
             constexpr int y = decltype(yc)::value, pos = B.mass[ODD][y][s];
             if constexpr (pos >= 0) {
-                auto &acc = ODD ? R.yo[ODD ? y : 0] : R.ye[ODD ? 0 : y];
+                auto &acc = tile<ODD, y>(R);
                 acc = M::op(st.template get<pos>(), x, acc);
             }
         });
