@@ -16,7 +16,7 @@ int main()
         const auto truth = [](int t) { return t == 5 ? 5.0 : t == 4 ? 5.3 : t == 2 ? 5.6 : t == 1 ? 6.5 : 20.0; };
         int n = 0;
         // delays only make a timing longer; the first one runs at low clocks
-        const auto sample = [&](int t) { return truth(t) * (1 + 0.1 * u(rng) * u(rng) + (n++ == 0 ? 0.15 : 0.0)); };
+        const auto sample = [&](int t, int) { return truth(t) * (1 + 0.1 * u(rng) * u(rng) + (n++ == 0 ? 0.15 : 0.0)); };
         std::vector<double> times;
         const int t = pick_tile(cand, sample, &times);
         wrong += t != 5;
@@ -27,7 +27,7 @@ int main()
         int once = 0;
         double bt = 1e9;
         for (int c : cand) {
-            const double us = sample(c);
+            const double us = sample(c, 0);
             if (us < bt) bt = us, once = c;
         }
         wrong_once += once != 5;
@@ -35,11 +35,11 @@ int main()
     std::printf("wrong: %d of 200, with one timing each %d\n", wrong, wrong_once);
     if (wrong != 0 || wrong_once < 100) return std::puts("FAIL"), 1;
     // ties go to the earlier one; what cannot run is left out
-    if (pick_tile({3, 7}, [](int) { return 2.0; }) != 3) return std::puts("FAIL: tie"), 1;
+    if (pick_tile({3, 7}, [](int, int) { return 2.0; }) != 3) return std::puts("FAIL: tie"), 1;
     std::vector<double> times;
-    if (pick_tile({3, 7}, [](int t) { return t == 3 ? -1.0 : 2.0; }, &times) != 7 || times[0] < 1e300)
+    if (pick_tile({3, 7}, [](int t, int) { return t == 3 ? -1.0 : 2.0; }, &times) != 7 || times[0] < 1e300)
         return std::puts("FAIL: candidate that cannot run"), 1;
-    if (pick_tile({3}, [](int) { return -1.0; }) != -1) return std::puts("FAIL: none runs"), 1;
+    if (pick_tile({3}, [](int, int) { return -1.0; }) != -1) return std::puts("FAIL: none runs"), 1;
     std::puts("OK");
     return 0;
 }
