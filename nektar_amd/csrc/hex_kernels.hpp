@@ -764,8 +764,10 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_grouped_kernel(int co
 // Solver form: x gathered from the global vector of the structured n^3
 // mesh, element results written element-major (assembled afterwards); FP64:
 // edot[e] = x_e . y_e, its lines' sums added in the order of their indices.
+// by_xcd: one contiguous part of the elements per XCD (gather_by_xcd).
 template <typename T, int NM, int NQ, int EPB>
-__global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_gather_kernel(int n, int N, const T *__restrict__ tabp,
+__global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_gather_kernel(int n, int N, bool by_xcd,
+                                                                         const T *__restrict__ tabp,
                                                                          const T *__restrict__ geo, T lambda,
                                                                          const T *__restrict__ xg,
                                                                          T *__restrict__ out,
@@ -778,7 +780,7 @@ __global__ __launch_bounds__(EPB * NQ * NQ) void helmholtz_gather_kernel(int n, 
     const Tab<T, NM, NQ> tab{tabp};
     const int le = threadIdx.x / TPE, t = threadIdx.x % TPE;
     const int nelmt = n * n * n;
-    const int e = xcd_work(blockIdx.x, (nelmt + EPB - 1) / EPB) * EPB + le;
+    const int e = (by_xcd ? xcd_work(blockIdx.x, (nelmt + EPB - 1) / EPB) : (int)blockIdx.x) * EPB + le;
     const bool valid = e < nelmt;
     const int ex = e % n, ey = (e / n) % n, ez = e / (n * n);
     const StructuredFetch<T, NM> f{xg, N, ex * (NM - 1), ey * (NM - 1), ez * (NM - 1)};

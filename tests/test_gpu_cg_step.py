@@ -76,3 +76,13 @@ def test_true_residual_of_every_tile(nmf, nm, d, perturb):
             check_true_residual(s, n, nm, mixed=True)
         with pytest.raises(nmf.NektarError):
             s.set_tiles(3 if nm not in (9, 10) else 5, 0)
+
+
+@pytest.mark.parametrize("n,nm,mixed", [(35, 5, True), (36, 5, True), (44, 5, False), (45, 5, False)])
+def test_true_residual_around_the_cache(nmf, n, nm, mixed):
+    """Perturbed elements whose per-point geometry (7 values per point) is just
+    below and just above the 256 MB (FP32) and 1 GB (FP64) from which the
+    gather deals its workgroups to the XCDs in another order."""
+    size = n ** 3 * 7 * (nm + 1) ** 3 * (4 if mixed else 8) / 2 ** 20
+    assert (size > (256 if mixed else 1024)) == (n in (36, 45))
+    check_true_residual(nmf.HelmholtzSolver(n, nm, nm + 1, 1.3, perturb=0.1, seed=3), n, nm, mixed)
