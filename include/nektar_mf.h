@@ -218,7 +218,8 @@ int nmf_operator_apply_physderiv_host(nmf_operator op, const double *in,
  * instantiated for several tiles (elements per workgroup) and every tet
  * kernel for two (work-items per element: nq0*(nq0-1), elements sharing
  * waves, or that rounded up to a multiple of 64, one element per wave at
- * nq0 <= 8), and the fastest is measured per (key, nummodes, numpoints,
+ * nq0 <= 8; affine Helmholtz takes both and runs one kernel), and the
+ * fastest is measured per (key, nummodes, numpoints,
  * precision) on the caller's data.  The choice is remembered for the rest of
  * the process: operators and solvers created later for the same kind, with at
  * most four times the elements, start from it.
@@ -245,8 +246,8 @@ int nmf_operator_autotune(nmf_operator op, void *stream, int *tile,
  * collections in ExpList::GeneralMatrixOp (MultiRegions/ExpList.cpp:
  * 2666-2757: one Collection::ApplyOperator per shape/order collection)
  * with one submission: Helmholtz entries of one kind (shape, nummodes,
- * numpoints, precision, geometry type, tile) run as a single grouped
- * launch, kinds are spread over `streams` streams, and the whole batch is
+ * numpoints, precision, geometry type, the tile that runs) run as a single
+ * grouped launch, kinds are spread over `streams` streams, and the whole batch is
  * captured once into a hipGraph that every later run replays
  * (NMF_BATCH_GRAPH, the default).  NMF_BATCH_GROUPED launches the same
  * grouped kernels without a graph; NMF_BATCH_PER_ITEM applies entry by

@@ -24,13 +24,13 @@
 //   along q: S S, S R, R S  -> 3 slabs
 //   along r: u, d0, d1, d2 in registers, the metric, and the transposes back.
 // About 40 operations per coefficient against 183 with the contractions over
-// NQ points, and 20 LDS accesses against 33: bound by LDS (its pipe is busy 75 %
-// of the time at NM = 7), then HBM.  Measured against the contractions over
-// the points: 32,768 elements at NM = 7, NQ = 8, FP64 90.4 -> 52.5 us (3.5 TB/s
-// of the coefficients and geometry), 50,021 elements at NM = 4, NQ = 6, FP32
-// 29.3 -> 8.3 us.  Rounding error against extended precision 1.8e-16 at NM = 3,
-// 5, 7 and 10 (relative, 2-norm), the sums over the points 5.6, 5.3, 6.7 and
-// 33e-16.
+// NQ points, and 20 LDS accesses against 33: bound by LDS (its pipe is busy
+// 84 % of the cycles at NM = 7, a quarter of it bank conflicts), then HBM.
+// Measured against the contractions over the points: 32,768 elements at NM = 7,
+// NQ = 8, FP64 90.4 -> 52.5 us (3.5 TB/s of the coefficients and geometry),
+// 50,021 elements at NM = 4, NQ = 6, FP32 29.3 -> 8.3 us.  Rounding error
+// against extended precision 1.8e-16 at NM = 3, 5, 7 and 10 (relative, 2-norm),
+// the sums over the points 5.6, 5.3, 6.7 and 33e-16.
 #pragma once
 
 #include <hip/hip_runtime.h>

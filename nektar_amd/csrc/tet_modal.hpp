@@ -24,12 +24,11 @@
 // vectors never leave the registers.  The matrices come as a stream of 16x4
 // blocks in the order of use.
 //
-// Bound: the matrix cores (64 cycles a block in FP64, 32 in FP32; about 80 and
-// 45 measured with the metric's vector operations, which share the FP64 pipe)
-// and, in front and behind, the scattered coefficient accesses of a wave
-// (a quarter of the time at NM = 7).  Measured against sum factorisation on the vector
-// units, 32,768 elements at NM = 7, FP64: 125.7 -> 27 us; 4,001 elements at
-// NM = 10, FP32: 32.9 -> 13.6 us.
+// Bound: the matrix cores (64 cycles a block in FP64, 32 in FP32; busy 55 % and
+// 46 % of the cycles at NM = 7) and, in front and behind, the scattered
+// coefficient accesses of a wave, which nothing hides.  Measured against sum
+// factorisation on the vector units, 32,768 elements at NM = 7, FP64: 125.7 ->
+// 27 us; 4,001 elements at NM = 10, FP32: 32.9 -> 13.6 us.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -39,8 +39,7 @@ HEX = [((3, 4, 5), (4, 5, 6), 37), ((4, 4, 4), (6, 5, 7), 20), ((6, 3, 4), (9, 4
        ((11, 9, 10), (13, 13, 13), 1100)]
 TET = [((3, 4, 5), (5, 5, 5), 37), ((2, 3, 4), (4, 6, 5), 21), ((4, 4, 4), (6, 4, 7), 19),
        ((5, 5, 5), (7, 7, 7), 16), ((11, 11, 11), (12, 11, 11), 10), ((8, 10, 12), (16, 14, 14), 1030)]
-# prisms always run the runtime-size kernels: the MODIFIED defaults (P=3, 6,
-# 9), anisotropic sizes, and a size from the global workspace with more
+# prisms: the MODIFIED defaults (P=3 and 6, compile-time sizes, and 9), anisotropic sizes, and a size from the global workspace with more
 # elements than workgroups
 PRISM = [((4, 4, 4), (5, 5, 4), 37), ((7, 7, 7), (8, 8, 7), 64), ((3, 4, 5), (5, 4, 5), 15),
          ((4, 2, 4), (5, 6, 5), 33), ((10, 10, 10), (11, 11, 10), 12), ((12, 12, 12), (14, 14, 13), 1030)]
