@@ -1,5 +1,6 @@
 #include "tune.hpp"
 
+#include <cstdint>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -34,7 +35,7 @@ int tuned_tile(const TuneKey &k, int nelmt)
     const auto larger = by_count.lower_bound(nelmt);
     if (larger != by_count.end()) return larger->second;
     const auto &largest = *by_count.rbegin();
-    return nelmt / kTunedReach <= largest.first ? largest.second : 0;
+    return nelmt <= (int64_t)kTunedReach * largest.first ? largest.second : 0;
 }
 
 void record_tile(const TuneKey &k, int nelmt, int tile)

@@ -115,6 +115,8 @@ def test_recorded_choice_reaches_four_times_the_elements(nmf):
     assert best > 0 and small.tile == best
     assert op(3).tile == best and op(6).tile == best  # 27 and 216 of 64 elements
     assert op(7).tile == 0                            # 343
+    for n, want in ((256, best), (257, 0)):
+        assert nmf.GetOperatorFactory().CreateInstance("Helmholtz_Hex_Regular", 4, 5, n).tile == want
     large = op(12)
     large.tile = 0
     best_large, _ = large.autotune()
